@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -60,6 +61,25 @@ struct AdjArgs {
     int weno5;       // the WENO5-JS extension instead of the reference 'weno'
     int ntx, nty, nwork;  // set by the launcher
 };
+
+// Compute units of the current device.
+inline int device_cus()
+{
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
+        ncu = 256;
+    return ncu;
+}
+
+// Levels per work item of a column-marching kernel on `tiles` column tiles: as
+// many as still give `per_cu` work items per CU, within [least, most].
+inline int levels_per_item(int nz, long tiles, int per_cu, int least, int most)
+{
+    const long want = (long)per_cu * device_cus();
+    const long levels = (tiles * nz + want - 1) / want;
+    return (int)std::min<long>(nz, std::max<long>(least, std::min<long>(most, levels)));
+}
 
 // Launchers (scalar_fp64.hip, momentum_fp64.hip, util.hip, adjoint.hip).
 hipError_t launch_adjoint_stage(const AdjArgs &a, hipStream_t s);

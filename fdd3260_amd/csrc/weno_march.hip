@@ -28,35 +28,13 @@
 // Compiled with -ffp-contract=off.
 #include <algorithm>
 
+#include "fp64_div.hpp"
 #include "mimadv_internal.hpp"
 #include "weno_ratio.hpp"
 
 namespace mimadv {
 
 namespace {
-
-// FP64 division in the steps the compiler emits for n / d on gfx950
-// (reciprocal estimate, two Newton steps, quotient, residual, corrected
-// quotient) without its operand scaling and special-value fix-up.  Those
-// two steps leave operands and result unchanged when n, d and n/d are
-// normal numbers well inside the exponent range, so within that range the
-// result is the correctly rounded quotient, bit for bit the same as n / d
-// (checked on 3.4e10 random operand pairs in [2^-400, 2^400]).  A
-// reciprocal serves every quotient with the same denominator.
-__device__ __forceinline__ double refined_rcp(double d)
-{
-    double r = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-d, r, 1.0);
-    return fma(r, e, r);
-}
-
-__device__ __forceinline__ double quot(double n, double d, double r)
-{
-    const double q = n * r;
-    return fma(fma(-d, q, n), r, q);
-}
 
 // n / 6, correctly rounded, from the correctly rounded reciprocal y of 6:
 // q = n y is within an ulp of n/6 and q + (n - 6 q) y rounds to n / 6
