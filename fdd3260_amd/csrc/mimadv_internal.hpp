@@ -72,13 +72,16 @@ inline int device_cus()
     return ncu;
 }
 
-// Levels per work item of a column-marching kernel on `tiles` column tiles: as
-// many as still give `per_cu` work items per CU, within [least, most].
-inline int levels_per_item(int nz, long tiles, int per_cu, int least, int most)
+// Levels per work item of a column-marching kernel on `tiles` column tiles:
+// the columns are cut into as many chunks as keep the items within `per_cu`
+// per CU (whole rounds of resident items, none nearly empty), their length
+// within [1, most].  A small grid thereby marches short chunks on many CUs
+// instead of long ones on few.
+inline int levels_per_item(int nz, long tiles, int per_cu, int most)
 {
-    const long want = (long)per_cu * device_cus();
-    const long levels = (tiles * nz + want - 1) / want;
-    return (int)std::min<long>(nz, std::max<long>(least, std::min<long>(most, levels)));
+    const long chunks = std::max<long>(1, (long)per_cu * device_cus() / tiles);
+    const long levels = (nz + chunks - 1) / chunks;
+    return (int)std::min<long>(nz, std::max<long>(1, std::min<long>(most, levels)));
 }
 
 // Launchers (scalar_fp64.hip, momentum_fp64.hip, util.hip, adjoint.hip).
@@ -98,8 +101,8 @@ struct PosArgs {
 };
 hipError_t launch_positive_stage(const GridDev &g, const SchemeParams &sp, const PosArgs &a, hipStream_t s);
 // column-marching kernels (weno_march.hip): 'weno', WENO5, MUSCL, QUICK,
-// Lax-Wendroff and the unlimited forms; kchunk 0 = default
-hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int kchunk, hipStream_t s);
+// Lax-Wendroff and the unlimited forms
+hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s);
 hipError_t launch_momentum_fp64(const GridDev &g, int mom_ord, int lavisc, int ntime, const double *mu,
                                 const double *mv, const double *mw, const double *ut, const double *vt,
                                 const double *wt, double *ua, double *va, double *wa, hipStream_t s);

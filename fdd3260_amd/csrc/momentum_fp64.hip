@@ -118,7 +118,7 @@ constexpr int MOM_LEVELS = 16;
 //
 // Measured, mom_ord 4 with viscosity, against one thread per cell that
 // recomputes every flux from global memory with full divisions: 256x256x128
-// 2300 -> 280 us (2.2 TB/s of its 72 B per cell), 64x64x48 86 -> 24 us.
+// 2300 -> 280 us (2.2 TB/s of its 72 B per cell), 64x64x48 86 -> 22 us.
 template <int TX, int TY, bool VISC, bool EVEN>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(3, 8))) void momentum_march_kernel(
     GridDev g, MomCoefs c, const double *__restrict__ mu, const double *__restrict__ mv, const double *__restrict__ mw,
@@ -592,9 +592,9 @@ hipError_t launch_tile(const GridDev &g, const MomCoefs &c, const double *mu, co
     const int ntx = (g.nx - 5 + TX - 1) / TX, nty = TY > 1 ? (g.ny - 5 + TY - 1) / TY : 1;
     // Two rounds of resident items fill the device and overlap the start of one
     // item with the levels of others: 16-level items take 280 us at 256x256x128
-    // against 333 us for 43 levels (one round exactly), 2-level items 25 us at
+    // against 333 us for 43 levels (one round exactly), 1-level items 22 us at
     // 64x64x48 against 49 us for 8 levels.
-    const int kchunk = levels_per_item(g.nz, (long)ntx * nty, 2 * MOM_GROUPS, 2, MOM_LEVELS);
+    const int kchunk = levels_per_item(g.nz, (long)ntx * nty, 2 * MOM_GROUPS, MOM_LEVELS);
     const int nwork = ntx * nty * ((g.nz + kchunk - 1) / kchunk);
     hipLaunchKernelGGL((momentum_march_kernel<TX, TY, VISC, EVEN>), dim3(nwork), dim3(TX * TY), 0, s, g, c, mu, mv, mw, ut, vt, wt,
                        g.zm.dzw, g.zm.dz1w, g.zm.dz1, ua, va, wa, kchunk, ntx, nwork);

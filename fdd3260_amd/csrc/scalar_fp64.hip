@@ -235,7 +235,7 @@ hipError_t launch_scalar_fp64(const GridDev &g, const SchemeParams &sp, const Sc
 {
     switch (sp.scheme) {
     case 1: return launch_scheme<1>(g, sp, a, s);
-    case 0: case 2: case 3: case 4: case 5: case 6: case 7: return launch_march(g, sp, a, 0, s);
+    case 0: case 2: case 3: case 4: case 5: case 6: case 7: return launch_march(g, sp, a, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -494,13 +494,11 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     march_body<TX, TY, S>(g, sp, a, kchunk, ntx, nwork);
 }
 
-template <int TX, int TY, int S, int KC>
+template <int TX, int TY, int S>
 hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int kchunk, hipStream_t s)
 {
     const int ntx = (g.nx - 5 + TX - 1) / TX;
     const int nty = TY > 1 ? (g.ny - 5 + TY - 1) / TY : 1;
-    if (kchunk <= 0) kchunk = KC;
-    if (kchunk > g.nz) kchunk = g.nz;
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
     const int nwork = ntx * nty * nchunk;
     if constexpr (S == 3)
@@ -516,16 +514,28 @@ hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarArg
 }
 
 // Tiles, measured at 256x256x128 before the VGPR cap of the reference-weno
-// instance: the reference 'weno' on 32x8 columns with 8-level chunks (217 us
-// per launch; 64x4 took 228: 2.27 x/y faces per cell instead of 2.16 and a
-// wider halo), WENO5 on 16x16 with 16-level chunks (285 us; 32x8 takes 308,
-// 64x4 323).  Tiles of 512 threads are slower (fewer waves per SIMD).
-// The line schemes use the reference-weno tiles.
-template <int S, int TX3, int TY3, int KC3>
-hipError_t launch_dims(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int kchunk, hipStream_t s)
+// instance: the reference 'weno' on 32x8 columns (217 us per launch; 64x4 took
+// 228: 2.27 x/y faces per cell instead of 2.16 and a wider halo), WENO5 on
+// 16x16 (285 us; 32x8 takes 308, 64x4 323).  Tiles of 512 threads are slower
+// (fewer waves per SIMD).  The line schemes use the reference-weno tiles.
+//
+// Levels per item: a level is a serial chain of loads, faces and two barriers
+// (4 us in 3D, 2.4 us on the single-wave 2D tiles), so short chunks on all CUs
+// beat long ones on a few; the start of a chunk costs about one level.  32x8
+// tiles take one round of the four resident groups per CU, at most 8 levels:
+// 'weno' 55 -> 13 us at 64x64x48 (1 level; 8 before), 67 -> 41 us at
+// 139x117x75 (6), unchanged at 256x256x128 (8).  WENO5's longer levels are
+// better balanced by two rounds: 113 -> 64 us at 139x117x75 (3 levels; 16
+// before; one round takes 68).  2D tiles are one wave each, 16 per CU: 38 -> 7
+// us at 128x128 (1 level; 16 before).
+template <int S, int TX3, int TY3>
+hipError_t launch_dims(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
 {
-    if (g.ny > 1) return launch_tile<TX3, TY3, S, KC3>(g, sp, a, kchunk, s);
-    return launch_tile<64, 1, S, 16>(g, sp, a, kchunk, s);
+    constexpr int MOST = 8;
+    const long ntx3 = (g.nx - 5 + TX3 - 1) / TX3, nty3 = (g.ny - 5 + TY3 - 1) / TY3;
+    if (g.ny > 1)
+        return launch_tile<TX3, TY3, S>(g, sp, a, levels_per_item(g.nz, ntx3 * nty3, S == 3 ? 8 : 4, MOST), s);
+    return launch_tile<64, 1, S>(g, sp, a, levels_per_item(g.nz, (g.nx - 5 + 63) / 64, 16, MOST), s);
 }
 
 }  // namespace
@@ -660,16 +670,16 @@ hipError_t launch_positive_stage(const GridDev &g, const SchemeParams &sp, const
     return hipGetLastError();
 }
 
-hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int kchunk, hipStream_t s)
+hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
 {
     switch (sp.scheme) {
-    case 0: return launch_dims<0, 32, 8, 8>(g, sp, a, kchunk, s);
-    case 3: return launch_dims<3, 16, 16, 16>(g, sp, a, kchunk, s);
-    case 2: return launch_dims<2, 32, 8, 8>(g, sp, a, kchunk, s);
-    case 4: return launch_dims<4, 32, 8, 8>(g, sp, a, kchunk, s);
-    case 5: return launch_dims<5, 32, 8, 8>(g, sp, a, kchunk, s);
-    case 6: return launch_dims<6, 32, 8, 8>(g, sp, a, kchunk, s);
-    case 7: return launch_dims<7, 32, 8, 8>(g, sp, a, kchunk, s);
+    case 0: return launch_dims<0, 32, 8>(g, sp, a, s);
+    case 3: return launch_dims<3, 16, 16>(g, sp, a, s);
+    case 2: return launch_dims<2, 32, 8>(g, sp, a, s);
+    case 4: return launch_dims<4, 32, 8>(g, sp, a, s);
+    case 5: return launch_dims<5, 32, 8>(g, sp, a, s);
+    case 6: return launch_dims<6, 32, 8>(g, sp, a, s);
+    case 7: return launch_dims<7, 32, 8>(g, sp, a, s);
     default: return hipErrorInvalidValue;
     }
 }

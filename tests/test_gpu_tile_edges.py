@@ -35,3 +35,20 @@ def test_momentum_tile_edges(cuda, dims, bc, ntime, lavisc):
         a.stream_sync()
         for c in (0, 1, 2) if my else (0, 2):
             assert np.array_equal(outs[c].cpu().numpy(), ref[c]), f"component {c}"
+
+
+@pytest.mark.parametrize("scheme", ["weno", "weno5", "muscl"])
+@pytest.mark.parametrize("dims", [(139, 117, 75), (6, 6, 8), (33, 9, 8), (300, 0, 41), (1500, 0, 301)])
+def test_scalar_chunk_lengths(cuda, scheme, dims):
+    """Grids for which the dispatch takes one level per item, a few (with a
+    shorter last chunk) and several; the other tests' grids take one."""
+    print(f"case chunks {scheme} {dims}", flush=True)
+    mx, my, nz = dims
+    g, u, v, w, q = case3d(mx, my, nz) if my else case2d(mx, nz)
+    ref = np.zeros(g.shape)
+    Oracle(g, scal_adv=scheme, muscllimiter="VL").scalar_tendency(1.0, u, v, w, q, ref)
+    with Advection(g, scal_adv=scheme, muscllimiter="VL") as a:
+        du, dv, dw, dq, dx = _dev(cuda, u, v, w, q, np.zeros(g.shape))
+        a.scalar_tendency(1.0, du, dv, dw, [dq], [dx])
+        a.stream_sync()
+        assert np.array_equal(dx.cpu().numpy(), ref)
