@@ -36,6 +36,17 @@ __device__ __forceinline__ double quot(double n, double d, double r)
 // or NaN gives a NaN residual.
 constexpr int RES_BAD = 0x3 | 0x204 | 0x90;
 
+// n / d with the refined reciprocal where the steps are exact, the plain
+// division elsewhere (see refined_rcp, RES_BAD); exact zeros may lose their
+// sign.
+__device__ __forceinline__ double quotient(double n, double d)
+{
+    const double r = refined_rcp(d), q = n * r, e = fma(-d, q, n), a = fabs(d);
+    double v = fma(e, r, q);
+    if (__builtin_expect(!(a >= 0x1p-400 && a <= 0x1p400) || __builtin_amdgcn_class(e, RES_BAD), 0)) v = n / d;
+    return v;
+}
+
 // Divisions by one positive denominator (a level thickness): one refined
 // reciprocal, then three instructions and a class test per numerator.  A
 // denominator outside the range of refined_rcp gets a NaN reciprocal, which

@@ -62,6 +62,10 @@ struct AdjArgs {
     int ntx, nty, nwork;  // set by the launcher
 };
 
+// Forms v here: keeps the scheduler from overlapping two register-hungry parts
+// of a kernel.
+__device__ __forceinline__ void settle(double &v) { asm volatile("" : "+v"(v) : : "memory"); }
+
 // Compute units of the current device.
 inline int device_cus()
 {

@@ -21,9 +21,6 @@ namespace mimadv {
 namespace {
 
 constexpr double AVISC = 1.0 / 16.0;
-// Forms v here: the scheduler otherwise overlaps the components of a cell,
-// and their operands do not fit the registers together.
-__device__ __forceinline__ void settle(double &v) { asm volatile("" : "+v"(v) : : "memory"); }
 constexpr int MOM_GROUPS = 3;  // resident work items per CU
 
 struct MomCoefs {

@@ -1,6 +1,6 @@
-// scalar_fp64.hip -- plain per-field FP64 scalar advection on gfx950: the
-// per-plane PPM kernel and the scheme dispatch (the other schemes run on the
-// column-marching kernels of weno_march.hip).
+// scalar_fp64.hip -- plain per-field FP64 scalar advection on gfx950: the PPM
+// kernel and the scheme dispatch (the other schemes run on the kernels of
+// weno_march.hip).
 //
 // One launch computes the fused x+y+z flux divergence of one field
 // (advection_x/y/z of src/TOOLS/advection.f90:556-798 for all three
@@ -9,232 +9,356 @@
 // with the periodic ghost images written in the same pass (so no separate
 // statebc/qnbc_p4 sweep is needed between stages).
 //
-// Work mapping: a workgroup of TX x TY threads owns a TX x TY tile of one
-// k-plane.  The plane tile plus a 3-cell halo in x and y is staged in LDS
-// with coalesced x-fastest loads.  The x and y cell records (Flux_r,
-// Flux_l of limiter_ppm and the CW84 averages) of the tile's cells and one
-// neighbour on each side are computed once each into LDS, and every cell
-// takes its x and y fluxes from them; the z records of levels k-1..k+1 come
-// from the thread's own column (coalesced across the wavefront).  Tiles for neighbouring k of the same
-// (x,y) tile have linear block ids 256-apart-multiples, so they land on the
-// same XCD and share its L2 for the column reads.
-//
 // This file is compiled with -ffp-contract=off: the arithmetic follows the
 // reference operation order and matches the CPU restatement bit for bit.
 #include "mimadv_internal.hpp"
 
 namespace mimadv {
 
-// z contribution of cell k (PPM)
-template <int SCHEME, class QF, class WF>
-__device__ __forceinline__ double z_contrib(int k, int nz, bool adv, const GridDev &g, const SchemeParams &sp,
-                                            QF Q, WF W)
-{
-    static_assert(SCHEME == 1, "per-plane kernel: PPM only");
-    const ZMetrics &zm = g.zm;
-    int bc5 = g.bcl[4], bc6 = g.bcl[5];
-    double bc51 = (bc5 == 0) ? 1.0 : 0.0, bc61 = (bc6 == 0) ? 1.0 : 0.0;
-    // cells k-1, k, k+1 (level nz carries only its Flux_l)
-    PPMRec cm{0.0, 0.0}, c0{0.0, 0.0}, cp{0.0, 0.0};
-    auto cell = [&](int c) -> PPMRec {
-        if (c == nz) {
-            PPMRec r;
-            r.fr = 0.0;
-            r.fl = ppm_ztop_fl(nz, zm, sp, Q, W);
-            return r;
-        }
-        return ppm_zcell(c, nz, zm, sp, bc51, bc61, Q, W);
-    };
-    bool need = (k >= 2 && k <= nz - 1) || (k == 1 && bc5 == 1) || (k == nz && bc6 == 1);
-    if (!need) return 0.0;
-    if (k >= 2) cm = cell(k - 1);
-    c0 = cell(k);
-    if (k <= nz - 1) cp = cell(k + 1);
-    auto face = [&](int f) -> double {
-        if (f == k - 1) return ppm_faceflux(cm.fr, c0.fl, W(k));
-        return ppm_faceflux(c0.fr, cp.fl, W(k + 1));
-    };
-    return z_assemble(k, nz, adv, bc5, bc6, zm, face, Q, W);
-}
+namespace {
 
-template <int SCHEME, int TX, int TY>
-__global__ __launch_bounds__(TX *TY) void scalar_fp64_kernel(GridDev g, SchemeParams sp, ScalarArgs a)
+// One work item: a TX x TY column tile marched up a chunk of levels.
+//
+// What bounds it: vector issue.  A cell record (limiter_ppm and the CW84
+// averages Flux_r, Flux_l) is about 130 instructions, so each is formed once:
+// per level the plane tile with a 3-cell halo and the face velocities go
+// through LDS, the x records of the cells i0-1..i0+TX of each row and the y
+// records of j0-1..j0+TY of each column are formed by a flattened loop over
+// the group, and the z record of level k+1 is formed once by its column's
+// thread and carried up (its differences, gammas and face value with it).
+// 3.3 records per cell; a chunk above the floor first forms two z records.
+// 128 VGPRs (a dozen loop-invariant offsets spill) give four groups per CU.
+//
+// Measured against one group per tile and level with 5.5 records per cell and
+// full divisions in the limiter (1670 vector instructions per cell, now 760):
+// 256x256x128 430 -> 280 us, 139x117x75 96 -> 63 us, 128x128 (2D) 11.6 -> 10.3
+// us.  32x8 tiles take 314 us, 144 VGPRs without spills (three groups) 300 us.
+template <int TX, int TY>
+__global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) void ppm_march_kernel(
+    GridDev g, SchemeParams sp, ScalarArgs a, int kchunk, int ntx)
 {
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
     constexpr bool THREE_D = TY > 1;
-    constexpr int NT = TX * TY;
-    constexpr int LW = TX + 6;
-    constexpr int LH = THREE_D ? TY + 6 : 1;
-    // cell records (Flux_r, Flux_l) of the x cells i0-1 .. i0+TX of each row
-    // and the y cells j0-1 .. j0+TY of each column, each computed once
+    constexpr int NT = TX * TY, H = 3;
+    constexpr int LW = TX + 2 * H, LH = THREE_D ? TY + 2 * H : 1, PL = LW * LH;
     constexpr int NXR = TY * (TX + 2), NYR = THREE_D ? (TY + 2) * TX : 0, NR = NXR + NYR;
-    __shared__ double tile[LH][LW];
+    // velocities: u(i0-1..i0+TX+1) of each row, v(j0-1..j0+TY+1) of each column
+    constexpr int UW = TX + 3, NU = TY * UW, NVEL = NU + (THREE_D ? (TY + 3) * TX : 0);
+    constexpr int TS = (PL + NT - 1) / NT, VS = (NVEL + NT - 1) / NT, RS = (NR + NT - 1) / NT;
+    __shared__ double tile[PL];
+    __shared__ double vel[NVEL];
     __shared__ double rfr[NR], rfl[NR];
 
-    const int k = blockIdx.z + 1;
-    const int i0 = 4 + blockIdx.x * TX;
-    const int j0 = THREE_D ? 4 + blockIdx.y * TY : 1;
+    const int nx = g.nx, ny = g.ny, nz = g.nz, mx = nx - 5, my = ny - 5;
     const size_t plane = (size_t)nx * ny;
-    const size_t kbase = (size_t)(k - 1) * plane;
-    const double *__restrict__ qk = a.q + kbase;
-    const int mx = nx - 5, my = ny - 5;  // interior extents (periodic images)
-
-    for (int t = threadIdx.y * TX + threadIdx.x; t < LH * LW; t += TX * TY) {
-        int r = t / LW, c = t - r * LW;
-        // positions outside the array are replaced by their periodic
-        // interior image; the PPM closures never read them
-        int ii = i0 - 3 + c;
-        if (ii < 1 || ii > nx) {
-            int rr = (ii - 4) % mx;
-            ii = (rr < 0 ? rr + mx : rr) + 4;
+    const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
+    const int nchunk = (nz + kchunk - 1) / kchunk;
+    const int tile_id = blockIdx.x / nchunk, kc = blockIdx.x - tile_id * nchunk;
+    const int i0 = 4 + (tile_id % ntx) * TX, j0 = THREE_D ? 4 + (tile_id / ntx) * TY : 1;
+    const int k0 = 1 + kc * kchunk, k1 = min(nz, k0 + kchunk - 1);
+    const int i = i0 + tx, j = j0 + ty;
+    const bool valid = i <= nx - 2 && (!THREE_D || j <= ny - 2);
+    unsigned col = 8u * (unsigned)((min(i, nx - 2) - 1) + nx * (THREE_D ? min(j, ny - 2) - 1 : 0));
+    const double dx1 = 1.0 / g.dx, dy1 = 1.0 / g.dy, dt0 = sp.dt0;
+    const bool adv = a.adv != 0, xdir = (a.dirmask & 1) != 0, ydir = THREE_D && (a.dirmask & 2),
+               zdir = (a.dirmask & 4) != 0;
+    const int bc5 = g.bcl[4], bc6 = g.bcl[5];
+    const double bc51 = bc5 == 0 ? 1.0 : 0.0, bc61 = bc6 == 0 ? 1.0 : 0.0;
+    const double *__restrict__ dz1w = g.zm.dz1w, *__restrict__ dz1 = g.zm.dz1, *__restrict__ ppmc = g.zm.ppmc;
+    const bool accum = a.epi == EPI_ACCUM, heun = a.epi == EPI_HEUN, so = a.epi == EPI_SO;
+    const bool need_tend = heun && a.b_lm != 0.0;
+    // the array the epilogue starts from: the tendency or the step-start state
+    const double *base = accum ? a.xs : (heun || so ? a.q0 : nullptr);
+    // positions past the array (padding of a partial tile) read a periodic
+    // image that feeds no interior cell
+    auto img = [](int x, int n, int m) { return x > n ? (x - 4) % m + 4 : x; };
+    unsigned toff[TS], voff[VS];
+#pragma unroll
+    for (int s = 0; s < TS; ++s) {
+        const int e = min(tid + s * NT, PL - 1), r = e / LW, c = e - r * LW;
+        toff[s] = 8u * (unsigned)((img(i0 - H + c, nx, mx) - 1) + (THREE_D ? nx * (img(j0 - H + r, ny, my) - 1) : 0));
+    }
+#pragma unroll
+    for (int s = 0; s < VS; ++s) {
+        const int e = min(tid + s * NT, NVEL - 1);
+        if (e < NU) {
+            const int r = e / UW, c = e - r * UW;
+            voff[s] = 8u * (unsigned)((img(i0 - 1 + c, nx, mx) - 1) + (THREE_D ? nx * (img(j0 + r, ny, my) - 1) : 0));
+        } else {
+            const int e2 = e - NU, r = e2 / TX, c = e2 - r * TX;
+            voff[s] = 8u * (unsigned)((img(i0 + c, nx, mx) - 1) + nx * (img(j0 - 1 + r, ny, my) - 1));
         }
-        int jj = 1;
-        if (THREE_D) {
-            jj = j0 - 3 + r;
-            if (jj < 1 || jj > ny) {
-                int rr = (jj - 4) % my;
-                jj = (rr < 0 ? rr + my : rr) + 4;
+    }
+    // record 3 or n-1 of a line lies in this item
+    const bool edge = i0 == 4 || i0 + TX > nx - 2 || (THREE_D && (j0 == 4 || j0 + TY > ny - 2));
+
+    // element at a 32-bit byte offset from a wave-uniform level plane
+    auto at = [&](const double *p, unsigned byte) {
+        return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + byte);
+    };
+    auto put = [&](double *p, unsigned byte, double v) {
+        *reinterpret_cast<double *>(reinterpret_cast<char *>(p) + byte) = v;
+    };
+    auto Q = [&](int kk) { return at(a.q + (size_t)(kk - 1) * plane, col); };
+    auto W = [&](int kk) { return kk >= 1 && kk <= nz ? at(a.w + (size_t)(kk - 1) * plane, col) : 0.0; };
+    // difference D(m) = Q(m+1) - Q(m); D(0), D(-1) and D(nz) are what the
+    // reference puts beyond a periodic (else closed) floor and lid, `near` =
+    // D(nz-1) the neighbour of the lid
+    auto below = [&](int m) { return bc51 * (m == 0 ? Q(nz - 4) - Q(nz - 5) : Q(nz - 5) - Q(nz - 6)); };
+    auto lid = [&](double near) { return bc61 * (Q(6) - Q(5)) + (1.0 - bc61) * near; };
+
+    // z state of iteration k, which forms the record of level c = k+1
+    const int kstart = zdir ? max(k0 - 2, 0) : k0;
+    double qm = 0.0, qc = 0.0, qp = 0.0;     // Q(c-1), Q(c), Q(c+1)
+    double dm2 = 0.0, dm1 = 0.0, d0 = 0.0;   // D(c-2), D(c-1), D(c)
+    double gm = 0.0, g0 = 0.0;               // ppm_gamma of (D(c-1), D(c-2)), (D(c), D(c-1))
+    double xlo = 0.0;                        // left face value of c
+    double wc = 0.0;                         // W(c)
+    double frk = 0.0, fzb = 0.0;             // Flux_r of level k, flux of face k-1
+    double qn = 0.0, wn = 0.0;               // Q(c+2), W(c+1), requested one level ahead
+    if (zdir) {
+        const int c = kstart + 1;
+        qc = Q(c);
+        qp = c < nz ? Q(c + 1) : 0.0;
+        wc = W(c);
+        d0 = c < nz ? qp - qc : 0.0;
+        if (c == 1) {
+            qm = qp;  // the reference passes x(2) as the lower neighbour
+            dm1 = below(0);
+            dm2 = below(-1);
+            xlo = qc - 0.5 * d0;
+        } else {
+            qm = Q(c - 1);
+            dm1 = qc - qm;
+            dm2 = c == 2 ? below(0) : qm - Q(c - 2);
+            if (c < nz) xlo = ppm_zxplus(c - 1, nz, ppmc, qm, dm2, dm1, d0);
+        }
+        gm = ppm_gamma(dm1, dm2);
+        g0 = ppm_gamma(d0, dm1);
+        qn = c + 2 <= nz ? Q(c + 2) : 0.0;
+        wn = W(c + 1);
+    } else {
+        qm = Q(k0);
+    }
+
+    // operands of level k, requested one level ahead
+    double tv[TS], vv[VS], basev = 0.0, tdv = 0.0;
+    auto fetch = [&](int k) {
+        const size_t kb = (size_t)(k - 1) * plane;
+        const double *qk = a.q + kb, *uk = a.u + kb, *vk = a.v + kb;
+#pragma unroll
+        for (int s = 0; s < TS; ++s) tv[s] = at(qk, toff[s]);
+#pragma unroll
+        for (int s = 0; s < VS; ++s) {
+            const bool isu = tid + s * NT < NU;
+            vv[s] = 0.0;
+            if (isu ? xdir : ydir) vv[s] = isu ? at(uk, voff[s]) : at(vk, voff[s]);
+        }
+        if (base) basev = at(base + kb, col);
+        if (need_tend) tdv = at(a.tend + kb, col);
+    };
+    fetch(k0);
+#pragma unroll 1
+    for (int k = kstart; k <= k1; ++k) {
+        // the offsets are opaque per level: otherwise every array's 64-bit
+        // address is hoisted out of the loop into registers of its own
+#pragma unroll
+        for (int s = 0; s < TS; ++s) asm volatile("" : "+v"(toff[s]));
+#pragma unroll
+        for (int s = 0; s < VS; ++s) asm volatile("" : "+v"(voff[s]));
+        asm volatile("" : "+v"(col));
+        double fzt = 0.0, wk = 0.0;  // flux of face k, W(k+1)
+        if (zdir) {
+            const int c = k + 1;
+            wk = wc;
+            double fr = 0.0, fl = 0.0, dp = 0.0, gp = 0.0, xhi = 0.0;
+            if (c < nz) {
+                dp = c + 1 < nz ? qn - qp : lid(d0);
+                gp = ppm_gamma(dp, d0);
+                xhi = ppm_zxplus(c, nz, ppmc, qc, dm1, d0, dp);
+                const double mup = fabs(wn) * dt0 * dz1[c - 1], muc = fabs(wc) * dt0 * dz1[c - 1];
+                const PPMRec r = ppm_cell(sp.ppm_limiter, qc, qp, qm, xhi, xlo, d0, dp, dm1, dm2, g0, gp, gm, mup, muc);
+                fr = r.fr;
+                fl = r.fl;
+            } else if (c == nz) {
+                // Flux_l of the top level (advq_ppm.f90:411-414)
+                const double muc = fabs(wc) * dt0 * dz1[nz - 1];
+                fl = qc + 0.5 * dm1 * (1.0 - muc);
+            }
+            if (k >= 1 && k < nz) fzt = ppm_faceflux(frk, fl, wc);
+            // to level k+1
+            frk = fr;
+            qm = qc;
+            qc = qp;
+            qp = qn;
+            dm2 = dm1;
+            dm1 = d0;
+            d0 = dp;
+            gm = g0;
+            g0 = gp;
+            xlo = xhi;
+            wc = wn;
+            if (k < k1) {
+                qn = c + 3 <= nz ? Q(c + 3) : 0.0;
+                wn = W(c + 2);
             }
         }
-        tile[r][c] = qk[(size_t)(ii - 1) + (size_t)nx * (jj - 1)];
-    }
-    __syncthreads();
-
-    // positions past the array (padding of a partial tile) read a periodic
-    // image; their records feed no interior cell
-    auto wrap_hi = [](int x, int n, int m) { return x > n ? (x - 4) % m + 4 : x; };
-    for (int e = threadIdx.y * TX + threadIdx.x; e < NR; e += NT) {
-        PPMRec rec;
-        if (e < NXR) {
-            if (!(a.dirmask & 1)) continue;
-            const int rr = e / (TX + 2), c = i0 - 1 + (e - rr * (TX + 2));
-            const int jr = THREE_D ? wrap_hi(j0 + rr, ny, my) : 1;
-            const double *__restrict__ urow = a.u + kbase + (size_t)nx * (jr - 1);
-            const int lr = THREE_D ? rr + 3 : 0;
-            auto Q = [&](int ii) { return tile[lr][ii - (i0 - 3)]; };
-            auto U = [&](int ii) { return urow[wrap_hi(ii, nx, mx) - 1]; };
-            rec = ppm_hcell(c, nx, 1.0 / g.dx, sp, Q, U);
-        } else {
-            if (!(THREE_D && (a.dirmask & 2))) continue;
-            const int e2 = e - NXR, rr = e2 / TX, cc = e2 - rr * TX, c = j0 - 1 + rr;
-            const double *__restrict__ vcol = a.v + kbase + (size_t)(wrap_hi(i0 + cc, nx, mx) - 1);
-            auto Q = [&](int jj) { return tile[jj - (j0 - 3)][cc + 3]; };
-            auto V = [&](int jj) { return vcol[(size_t)nx * (wrap_hi(jj, ny, my) - 1)]; };
-            rec = ppm_hcell(c, ny, 1.0 / g.dy, sp, Q, V);
+        if (k < k0) {
+            fzb = fzt;
+            continue;
         }
-        rfr[e] = rec.fr;
-        rfl[e] = rec.fl;
-    }
-    __syncthreads();
-
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i = i0 + tx, j = j0 + ty;
-    if (i > nx - 2 || (THREE_D && j > ny - 2)) return;
-    const size_t col = (size_t)(i - 1) + (size_t)nx * (j - 1);
-    const size_t id = col + kbase;
-    const bool adv = a.adv != 0;
-    const int lrow = THREE_D ? ty + 3 : 0;
-
-    double X = 0.0, Y = 0.0, Z = 0.0;
-    const double qc = tile[lrow][tx + 3];
-    if (a.dirmask & 1) {
-        // ppm_h (advq_ppm.f90:136-163) on the records of cells i-1, i, i+1
-        const double *__restrict__ urow = a.u + kbase + (size_t)nx * (j - 1);
-        const double d1 = 1.0 / g.dx, ui = urow[i - 1], uip = urow[i];
-        const int e = ty * (TX + 2) + tx;
-        double fr_i = rfr[e + 1], fl_ip = rfl[e + 2];
-        if (g.bcl[1] != 0 && i == nx - 2) {
-            fr_i = rfl[e + 1];  // Flux_r(ii2) = Flux_l(ii2)
-            fl_ip = rfr[e];     // Flux_l(ii2+1) = Flux_r(ii2-1)
+        // the z record is finished here (its temporaries do not fit the
+        // registers beside the rest)
+        settle(fzt);
+        settle(frk);
+        const size_t kb = (size_t)(k - 1) * plane;
+#pragma unroll
+        for (int s = 0; s < TS; ++s)
+            if (tid + s * NT < PL) tile[tid + s * NT] = tv[s];
+#pragma unroll
+        for (int s = 0; s < VS; ++s)
+            if (tid + s * NT < NVEL) vel[tid + s * NT] = vv[s];
+        const double basec = basev, tdc = tdv;
+        __syncthreads();
+        if (k < k1) fetch(k + 1);
+        // one record at a time: ppm_cell is register-hungry
+#pragma unroll 1
+        for (int s = 0; s < RS; ++s) {
+            const int e = tid + s * NT;
+            if (e >= NR) break;
+            int b, st, c, n;
+            double u0, u1, d1;
+            if (e < NXR) {
+                if (!xdir) continue;
+                const int r = e / (TX + 2), cc = e - r * (TX + 2);
+                b = (THREE_D ? r + H : 0) * LW + cc + 2;
+                st = 1;
+                c = i0 - 1 + cc;
+                n = nx;
+                u0 = vel[r * UW + cc];
+                u1 = vel[r * UW + cc + 1];
+                d1 = dx1;
+            } else {
+                if (!ydir) break;
+                const int e2 = e - NXR, r = e2 / TX, cc = e2 - r * TX;
+                b = (r + 2) * LW + cc + H;
+                st = LW;
+                c = j0 - 1 + r;
+                n = ny;
+                u0 = vel[NU + r * TX + cc];
+                u1 = vel[NU + (r + 1) * TX + cc];
+                d1 = dy1;
+            }
+            const double mup = fabs(u1) * dt0 * d1, muc = fabs(u0) * dt0 * d1;
+            const double m2 = tile[b - 2 * st], m1 = tile[b - st], x0 = tile[b], p1 = tile[b + st], p2 = tile[b + 2 * st];
+            const PPMRec r = edge ? ppm_hcell<true>(c, n, sp, m2, m1, x0, p1, p2, mup, muc)
+                                  : ppm_hcell<false>(c, n, sp, m2, m1, x0, p1, p2, mup, muc);
+            rfr[e] = r.fr;
+            rfl[e] = r.fl;
         }
-        const double flux_old = ppm_faceflux(rfr[e], rfl[e + 1], ui);
-        const double flux = ppm_faceflux(fr_i, fl_ip, uip);
-        X = (flux - flux_old) * d1;
-        if (adv) X = X - qc * (uip - ui) * d1;
-    }
-    if (THREE_D && (a.dirmask & 2)) {
-        const double *__restrict__ vcol = a.v + kbase + (size_t)(i - 1);
-        const double d1 = 1.0 / g.dy, vj = vcol[(size_t)nx * (j - 1)], vjp = vcol[(size_t)nx * j];
-        const int e = NXR + ty * TX + tx;
-        double fr_j = rfr[e + TX], fl_jp = rfl[e + 2 * TX];
-        if (g.bcl[3] != 0 && j == ny - 2) {
-            fr_j = rfl[e + TX];
-            fl_jp = rfr[e];
+        // what the cell takes from the tile and the velocities is read here: the
+        // next level's values go there as soon as the barrier is passed
+        const double qcell = tile[(THREE_D ? ty + H : 0) * LW + tx + H];
+        const double ui = vel[ty * UW + tx + 1], uip = vel[ty * UW + tx + 2];
+        double vj = 0.0, vjp = 0.0;
+        if constexpr (THREE_D) {
+            vj = vel[NU + (ty + 1) * TX + tx];
+            vjp = vel[NU + (ty + 2) * TX + tx];
         }
-        const double flux_old = ppm_faceflux(rfr[e], rfl[e + TX], vj);
-        const double flux = ppm_faceflux(fr_j, fl_jp, vjp);
-        Y = (flux - flux_old) * d1;
-        if (adv) Y = Y - qc * (vjp - vj) * d1;
-    }
-    if (a.dirmask & 4) {
-        const double *__restrict__ qc = a.q + col;
-        const double *__restrict__ wc = a.w + col;
-        auto Q = [&](int kk) { return qc[plane * (size_t)(kk - 1)]; };
-        auto W = [&](int kk) { return wc[plane * (size_t)(kk - 1)]; };
-        Z = z_contrib<SCHEME>(k, nz, adv, g, sp, Q, W);
-    }
-
-    if (a.epi == EPI_ACCUM || a.epi == EPI_OVERWRITE) {
-        double r = (a.epi == EPI_ACCUM) ? a.xs[id] : 0.0;
-        if (a.dirmask & 1) r = r - X;
-        if (THREE_D && (a.dirmask & 2)) r = r - Y;
-        if (a.dirmask & 4) r = r - Z;
-        a.xs[id] = r;
-        return;
-    }
-    double A = 0.0;
-    if (a.dirmask & 1) A = A - X;
-    if (THREE_D && (a.dirmask & 2)) A = A - Y;
-    if (a.dirmask & 4) A = A - Z;
-    double qn;
-    if (a.epi == EPI_HEUN) {
-        double T = (a.b_lm != 0.0) ? A + a.b_lm * a.tend[id] : A + 0.0;
-        a.tend[id] = T;
-        qn = a.q0[id] + a.adt * T;
-    } else {
-        qn = a.c0 * a.q0[id] + a.c1 * (a.q[id] + a.dt * A);
-    }
-    a.qn[id] = qn;
-    if (a.fill) {
-        // periodic images (qnbc_p4, bc.f90:409-414 and :431-436):
-        // x(1:3) = x(nx-4:nx-2), x(nx-1:nx) = x(4:5), same in y, corners
-        // from both
-        int ix = 0, jy = 0;
-        if (i >= nx - 4) ix = i - mx;
-        else if (i <= 5) ix = i + mx;
-        if (THREE_D) {
-            if (j >= ny - 4) jy = j - my;
-            else if (j <= 5) jy = j + my;
+        __syncthreads();
+        if (valid) {
+            double X = 0.0, Y = 0.0, Z = 0.0;
+            if (xdir) {
+                // ppm_h (advq_ppm.f90:136-163) on the records of cells i-1, i, i+1
+                const int e = ty * (TX + 2) + tx;
+                double fr_i = rfr[e + 1], fl_ip = rfl[e + 2];
+                if (g.bcl[1] != 0 && i == nx - 2) {
+                    fr_i = rfl[e + 1];  // Flux_r(ii2) = Flux_l(ii2)
+                    fl_ip = rfr[e];     // Flux_l(ii2+1) = Flux_r(ii2-1)
+                }
+                const double flux_old = ppm_faceflux(rfr[e], rfl[e + 1], ui);
+                X = (ppm_faceflux(fr_i, fl_ip, uip) - flux_old) * dx1;
+                if (adv) X = X - qcell * (uip - ui) * dx1;
+            }
+            if (ydir) {
+                const int e = NXR + ty * TX + tx;
+                double fr_j = rfr[e + TX], fl_jp = rfl[e + 2 * TX];
+                if (g.bcl[3] != 0 && j == ny - 2) {
+                    fr_j = rfl[e + TX];
+                    fl_jp = rfr[e];
+                }
+                const double flux_old = ppm_faceflux(rfr[e], rfl[e + TX], vj);
+                Y = (ppm_faceflux(fr_j, fl_jp, vjp) - flux_old) * dy1;
+                if (adv) Y = Y - qcell * (vjp - vj) * dy1;
+            }
+            if (zdir) {
+                // no-flux 'nnf' floor/lid, zero z tendency at other ends
+                if (k >= 2 && k < nz) {
+                    Z = (fzt - fzb) * dz1w[k - 1];
+                    if (adv) Z = Z - qcell * (wk - W(k)) * dz1w[k - 1];
+                } else if (k == 1 && bc5 == 1) {
+                    Z = 0.0 + (fzt - 0.0) * dz1w[0];
+                    if (adv) Z = Z - qcell * (wk - 0.0) * dz1w[0];
+                } else if (k == nz && bc6 == 1) {
+                    Z = 0.0 + (0.0 - fzb) * dz1w[nz - 1];
+                    if (adv) Z = Z - qcell * (0.0 - W(nz)) * dz1w[nz - 1];
+                }
+            }
+            double r = accum ? basec : 0.0;
+            if (xdir) r = r - X;
+            if (ydir) r = r - Y;
+            if (zdir) r = r - Z;
+            if (accum || a.epi == EPI_OVERWRITE) {
+                put(a.xs + kb, col, r);
+            } else {
+                double q;
+                if (heun) {
+                    const double T = need_tend ? r + a.b_lm * tdc : r + 0.0;
+                    put(a.tend + kb, col, T);
+                    q = basec + a.adt * T;
+                } else {
+                    q = a.c0 * basec + a.c1 * (qcell + a.dt * r);
+                }
+                put(a.qn + kb, col, q);
+                if (a.fill) {
+                    // periodic images (qnbc_p4, bc.f90:409-414 and :431-436)
+                    int ix = 0, jy = 0;
+                    if (i >= nx - 4) ix = i - mx;
+                    else if (i <= 5) ix = i + mx;
+                    if (THREE_D) {
+                        if (j >= ny - 4) jy = j - my;
+                        else if (j <= 5) jy = j + my;
+                    }
+                    double *qo = a.qn + kb;
+                    if (ix) qo[(size_t)(ix - 1) + (size_t)nx * (j - 1)] = q;
+                    if (jy) {
+                        qo[(size_t)(i - 1) + (size_t)nx * (jy - 1)] = q;
+                        if (ix) qo[(size_t)(ix - 1) + (size_t)nx * (jy - 1)] = q;
+                    }
+                }
+            }
         }
-        double *qk_out = a.qn + kbase;
-        if (ix) qk_out[(size_t)(ix - 1) + (size_t)nx * (j - 1)] = qn;
-        if (jy) {
-            qk_out[(size_t)(i - 1) + (size_t)nx * (jy - 1)] = qn;
-            if (ix) qk_out[(size_t)(ix - 1) + (size_t)nx * (jy - 1)] = qn;
-        }
+        fzb = fzt;
     }
 }
 
-template <int SCHEME>
-static hipError_t launch_scheme(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
+template <int TX, int TY>
+hipError_t launch_ppm(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int per_cu, hipStream_t s)
 {
-    int mxi = g.nx - 5;
-    if (g.ny > 1) {
-        constexpr int TX = 64, TY = 4;
-        dim3 grid((mxi + TX - 1) / TX, (g.ny - 5 + TY - 1) / TY, g.nz);
-        hipLaunchKernelGGL((scalar_fp64_kernel<SCHEME, TX, TY>), grid, dim3(TX, TY), 0, s, g, sp, a);
-    } else {
-        constexpr int TX = 64, TY = 1;
-        dim3 grid((mxi + TX - 1) / TX, 1, g.nz);
-        hipLaunchKernelGGL((scalar_fp64_kernel<SCHEME, TX, TY>), grid, dim3(TX, TY), 0, s, g, sp, a);
-    }
+    const int ntx = (g.nx - 5 + TX - 1) / TX, nty = TY > 1 ? (g.ny - 5 + TY - 1) / TY : 1;
+    const int kchunk = levels_per_item(g.nz, (long)ntx * nty, per_cu, 16);
+    const int items = ntx * nty * ((g.nz + kchunk - 1) / kchunk);
+    hipLaunchKernelGGL((ppm_march_kernel<TX, TY>), dim3(items), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx);
     return hipGetLastError();
 }
+
+}  // namespace
 
 hipError_t launch_scalar_fp64(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
 {
     switch (sp.scheme) {
-    case 1: return launch_scheme<1>(g, sp, a, s);
+    // one round of the resident groups: two rounds take 67 instead of 63 us at
+    // 139x117x75 and the same at 256x256x128
+    case 1: return g.ny > 1 ? launch_ppm<16, 16>(g, sp, a, 4, s) : launch_ppm<64, 1>(g, sp, a, 16, s);
     case 0: case 2: case 3: case 4: case 5: case 6: case 7: return launch_march(g, sp, a, s);
     default: return hipErrorInvalidValue;
     }

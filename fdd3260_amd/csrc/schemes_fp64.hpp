@@ -12,6 +12,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "fp64_div.hpp"
+#include "weno_ratio.hpp"
+
 namespace mimadv {
 
 struct ZMetrics {
@@ -344,61 +347,71 @@ __device__ __forceinline__ double lw_zface(int f, int nz, const ZMetrics &zm, co
 // PPM (advq_ppm.f90)
 // ---------------------------------------------------------------------------
 
-// sqrt(spacing(x)) of Fortran for REAL(8): spacing = 2**max(ilogb(x)-52,-1022)
-// (2**-1022 for x == 0); the square root of a power of two is exact or
-// sqrt(2) times one.
-__device__ __forceinline__ double sqrt_spacing(double x)
+// |x| > sqrt(spacing(x)) of Fortran for REAL(8), spacing = 2**(ilogb(x)-52)
+// (2**-1022 at least): the root is 2**((e-52)/2) for an even exponent e of x
+// and fl(sqrt(2)) 2**((e-53)/2) for an odd one, so it lies above |x| for e <=
+// -54, at fl(sqrt(2)) 2**-53 for e = -53, at 2**-52 for e = -52 and below |x|
+// from e = -51 on (false for infinities and NaN, whose root is infinite or
+// undefined).
+__device__ __forceinline__ bool above_sqrt_spacing(double x)
 {
-    int e = (x == 0.0) ? -1022 : ilogb(x) - 52;
-    if (e < -1022) e = -1022;
-    if ((e & 1) == 0) return ldexp(1.0, e / 2);
-    return ldexp(1.4142135623730951, (e - 1) / 2);
+    const double a = fabs(x);
+    return a > 0x1.6a09e667f3bcdp-53 && a != 0x1p-52 && a < __builtin_inf();
 }
 
 struct PPMRec {
     double fr, fl;
 };
 
-// limiter_ppm (advq_ppm.f90:449-530) followed by the CW84 face averages
-// Flux_r/Flux_l (advq_ppm.f90:93-94)
-__device__ __forceinline__ PPMRec ppm_cell(int use_lim, double xx, double xp, double xm, double xplus,
-                                           double xmin, double ffip1, double ffip2, double ffim1,
-                                           double ffim2, double mup, double muc)
+// smoothness of two neighbouring differences (advq_ppm.f90:449-530)
+__device__ __forceinline__ double ppm_gamma(double a, double b)
 {
-    const double eps = 1.e-15, thres = 10.0;
-    double rp1 = 1.0;
+    const double d = a - b, s = a + b;
+    return 0.5 * (d * d + s * s);
+}
+
+// limiter_ppm (advq_ppm.f90:449-530) followed by the CW84 face averages
+// Flux_r/Flux_l (advq_ppm.f90:93-94) of a cell: its value and neighbours, the
+// right and left face values, the four differences around it, gamma1..3 =
+// ppm_gamma of (ffip1, ffim1), (ffip2, ffip1), (ffim1, ffim2).  The
+// conditions are formed without short-circuits (a branch per term costs more
+// than the terms).
+__device__ __forceinline__ PPMRec ppm_cell(int use_lim, double xx, double xp, double xm, double xplus, double xmin,
+                                           double ffip1, double ffip2, double ffim1, double ffim2, double gamma1,
+                                           double gamma2, double gamma3, double mup, double muc)
+{
+    const double eps = 1.e-15;
     double phir = xplus, phil = xmin;
-    double g1a = ffip1 - ffim1, g1b = ffip1 + ffim1;
-    double g2a = ffip2 - ffip1, g2b = ffip2 + ffip1;
-    double g3a = ffim1 - ffim2, g3b = ffim1 + ffim2;
-    double gamma1 = 0.5 * (g1a * g1a + g1b * g1b);
-    double gamma2 = 0.5 * (g2a * g2a + g2b * g2b);
-    double gamma3 = 0.5 * (g3a * g3a + g3b * g3b);
-    double lambda = dmaxd(dmaxd(gamma1, gamma2), gamma3) / (dmind(dmind(gamma1, gamma2), gamma3) + eps);
+    // a NaN among the gammas comes with a NaN face value, which stays
+    const double gmax = fmax(fmax(gamma1, gamma2), gamma3), gmin = fmin(fmin(gamma1, gamma2), gamma3) + eps;
     double phi1 = phir - phil;
     double phi2 = 3.0 * (phil - 2.0 * xx + phir);
-    if (use_lim && lambda > thres) {
-        if (phir < 0.0 || ((phir - xx) * (xp - phir) < 0.0 &&
-                           (ffim1 * ffip2 >= 0.0 || ffim1 * ffip1 <= 0.0 || ffip2 * ffip1 <= 0.0))) {
-            phir = (fabs(phir - xx) < fabs(phir - xp)) ? xx : xp;
-        }
-        if (phil < 0.0 || ((xx - phil) * (phil - xm) < 0.0 &&
-                           (ffim2 * ffip1 >= 0.0 || ffim2 * ffim1 <= 0.0 || ffip1 * ffim1 <= 0.0))) {
-            phil = (fabs(phil - xx) < fabs(phil - xm)) ? xx : xm;
-        }
+    // lambda = gmax / gmin > 10 without the division
+    if (use_lim && ratio_above<10>(gmax, gmin)) {
+        const bool turn = ffip1 * ffim1 <= 0.0;
+        const bool wr = (phir < 0.0) | (((phir - xx) * (xp - phir) < 0.0) &
+                                        ((ffim1 * ffip2 >= 0.0) | turn | (ffip2 * ffip1 <= 0.0)));
+        const double nr = (fabs(phir - xx) < fabs(phir - xp)) ? xx : xp;
+        const bool wl = (phil < 0.0) | (((xx - phil) * (phil - xm) < 0.0) &
+                                        ((ffim2 * ffip1 >= 0.0) | (ffim2 * ffim1 <= 0.0) | turn));
+        const double nl = (fabs(phil - xx) < fabs(phil - xm)) ? xx : xm;
+        phir = wr ? nr : phir;
+        phil = wl ? nl : phil;
         phi1 = phir - phil;
         phi2 = 3.0 * (phil - 2.0 * xx + phir);
-        double slope = -0.5 * phi1 / (sgn1(phi2) * dmaxd(fabs(phi2), eps));
-        if (fabs(ffim1) > sqrt_spacing(ffim1)) rp1 = ffip1 / ffim1;
-        // (slope > -1/2 .or. slope < 1/2) holds for every non-NaN slope
-        if (fabs(phi2) > eps && (slope > -0.5 || slope < 0.5)) {
-            double lim = dmaxd(0.0, dmind(dmind(2.0, 0.5 * (rp1 + 1.0)), 2.0 * rp1));
-            phir = xx + 0.5 * ffim1 * lim;
-            phil = xx - 0.5 * ffim1 * lim;
-            if ((xx - phil) * (phir - xx) < 0.0) {
-                phil = xx;
-                phir = xx;
-            }
+        // slope = -phi1 / (2 sgn(phi2) max(|phi2|, eps)); the reference's
+        // (slope > -1/2 .or. slope < 1/2) holds for every slope but NaN,
+        // which takes phi1 NaN or an infinite phi1 over an infinite phi2
+        const double inf = __builtin_inf();
+        const bool slope_ok = (fabs(phi1) < inf) | ((phi1 == phi1) & (fabs(phi2) < inf));
+        if ((fabs(phi2) > eps) & slope_ok) {
+            // the ratio is finite or infinite here, not NaN
+            const double rp1 = above_sqrt_spacing(ffim1) ? quotient(ffip1, ffim1) : 1.0;
+            const double lim = fmax(0.0, fmin(fmin(2.0, 0.5 * (rp1 + 1.0)), 2.0 * rp1));
+            const double r = xx + 0.5 * ffim1 * lim, l = xx - 0.5 * ffim1 * lim;
+            const bool flat = (xx - l) * (r - xx) < 0.0;
+            phir = flat ? xx : r;
+            phil = flat ? xx : l;
             phi1 = phir - phil;
             phi2 = 0.0;
         }
@@ -409,43 +422,25 @@ __device__ __forceinline__ PPMRec ppm_cell(int use_lim, double xx, double xp, do
     return r;
 }
 
-// right-face value xplus of cell c on an x/y line (left boundary c = 3,
-// core c = 4..n-2), advq_ppm.f90:89,110
-template <class QF>
-__device__ __forceinline__ double ppm_hxplus(int c, QF Q)
+// Flux_r/Flux_l of cell c in 3..n-1 on an x/y line (advq_ppm.f90:79-134) from
+// its five values and the Courant numbers; EDGE: the tile touches a side, so
+// c may be 3 or n-1, whose closures take the nearer differences
+template <bool EDGE>
+__device__ __forceinline__ PPMRec ppm_hcell(int c, int n, const SchemeParams &sp, double qm2, double xm, double xx,
+                                            double xp, double qp2, double mup, double muc)
 {
-    if (c == 3) return Q(3) + 0.5 * (Q(4) - Q(3));
-    double ffip1 = Q(c + 1) - Q(c), ffip2 = Q(c + 2) - Q(c + 1), ffim1 = Q(c) - Q(c - 1);
-    double sl = 0.5 * (ffip1 + ffim1);
-    double slp1 = 0.5 * (ffip2 + ffip1);
-    return Q(c) + 0.5 * ffip1 - (1.0 / 6.0) * (slp1 - sl);
-}
-
-// Flux_r/Flux_l of cell c in 3..n-1 on an x/y line (advq_ppm.f90:79-134)
-template <class QF, class UF>
-__device__ __forceinline__ PPMRec ppm_hcell(int c, int n, double d1, const SchemeParams &sp, QF Q, UF U)
-{
-    double dt0 = sp.dt0;
-    double mup = fabs(U(c + 1)) * dt0 * d1;
-    double muc = fabs(U(c)) * dt0 * d1;
-    double xx = Q(c), xp = Q(c + 1), xm = Q(c - 1);
-    if (c == 3) {
-        double ffip1 = xp - xx, ffip2 = Q(5) - xp, ffim1 = xx - xm;
-        double xmin = 0.5 * (xp + xx);
-        double xplus = xx + 0.5 * ffip1;
-        return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim1, mup, muc);
-    }
-    double xmin = ppm_hxplus(c - 1, Q);
-    if (c == n - 1) {
-        double ffip1 = xp - xx, ffim1 = xx - xm, ffim2 = xm - Q(c - 2);
-        double xplus = xx + 0.5 * ffip1;
-        return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip1, ffim1, ffim2, mup, muc);
-    }
-    double ffip1 = xp - xx, ffip2 = Q(c + 2) - xp, ffim1 = xx - xm, ffim2 = xm - Q(c - 2);
-    double sl = 0.5 * (ffip1 + ffim1);
-    double slp1 = 0.5 * (ffip2 + ffip1);
-    double xplus = xx + 0.5 * ffip1 - (1.0 / 6.0) * (slp1 - sl);
-    return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim2, mup, muc);
+    const bool lo = EDGE && c == 3, hi = EDGE && c == n - 1;
+    const double ffip1 = xp - xx, ffim1 = xx - xm;
+    const double ffip2 = hi ? ffip1 : qp2 - xp, ffim2 = lo ? ffim1 : xm - qm2;
+    const double sl = 0.5 * (ffip1 + ffim1);  // also the slope of c-1 at its right
+    const double xr = xx + 0.5 * ffip1, xl = xm + 0.5 * ffim1;
+    double xplus = xr - (1.0 / 6.0) * (0.5 * (ffip2 + ffip1) - sl);
+    double xmin = xl - (1.0 / 6.0) * (sl - 0.5 * (ffim1 + ffim2));
+    if (lo | hi) xplus = xr;
+    if (EDGE && c == 4) xmin = xl;
+    if (lo) xmin = 0.5 * (xp + xx);
+    return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim2, ppm_gamma(ffip1, ffim1),
+                    ppm_gamma(ffip2, ffip1), ppm_gamma(ffim1, ffim2), mup, muc);
 }
 
 __device__ __forceinline__ double ppm_faceflux(double fr, double fl, double uf)
@@ -453,118 +448,22 @@ __device__ __forceinline__ double ppm_faceflux(double fr, double fl, double uf)
     return 0.5 * fr * (uf + fabs(uf)) + 0.5 * fl * (uf - fabs(uf));
 }
 
-// x/y contribution of cell i in 4..n-2 (advq_ppm.f90:136-163); bc_hi is the
-// east/north boundary code (non-periodic edge fix-up :143-146)
-template <class QF, class UF>
-__device__ __forceinline__ double ppm_h(int i, int n, double d1, bool adv, int bc_hi, const SchemeParams &sp,
-                                        QF Q, UF U)
-{
-    PPMRec cm = ppm_hcell(i - 1, n, d1, sp, Q, U);
-    PPMRec c0 = ppm_hcell(i, n, d1, sp, Q, U);
-    PPMRec cp = ppm_hcell(i + 1, n, d1, sp, Q, U);
-    double fr_i = c0.fr, fl_ip = cp.fl;
-    if (bc_hi != 0 && i == n - 2) {
-        fr_i = c0.fl;      // Flux_r(ii2) = Flux_l(ii2)
-        fl_ip = cm.fr;     // Flux_l(ii2+1) = Flux_r(ii2-1)
-    }
-    double flux_old = ppm_faceflux(cm.fr, c0.fl, U(i));
-    double flux = ppm_faceflux(fr_i, fl_ip, U(i + 1));
-    double t = (flux - flux_old) * d1;
-    if (adv) t = t - Q(i) * (U(i + 1) - U(i)) * d1;
-    return t;
-}
-
-// Per-level PPM coefficients (metric-only subexpressions of the non-uniform
-// face formula, advq_ppm.f90:379-383, evaluated in the same order):
+// Right-face value of level c (advq_ppm.f90:368-409) from its value x and the
+// differences D(c-1), D(c), D(c+1), D(m) = Q(m+1) - Q(m).  Per-level
+// coefficients (metric-only subexpressions of the non-uniform face formula,
+// advq_ppm.f90:379-383, evaluated in the same order):
 //  [0] delta/(dm1+delta+dp1)   [1] (2dm1+delta)/(dp1+delta)  [2] (delta+2dp1)/(dm1+delta)
 //  [3] dp1/(delta+dp1+dp2)     [4] (2delta+dp1)/(dp2+dp1)    [5] (dp1+2dp2)/(delta+dp1)
 //  [6] delta/(delta+dp1)       [7] 1/(dm1+delta+dp1+dp2)
 //  [8] 2dp1*delta/(delta+dp1)*((dm1+delta)/(2delta+dp1)-(dp2+dp1)/(2dp1+delta))
 //  [9] delta*(dm1+delta)/(2delta+dp1)   [10] dp1*(dp1+dp2)/(2dp1+delta)
-template <class QF>
-__device__ __forceinline__ double ppm_zxplus(int c, const ZMetrics &zm, QF Q)
+__device__ __forceinline__ double ppm_zxplus(int c, int nz, const double *ppmc, double x, double dm, double d, double dp)
 {
-    if (c <= 2) return Q(c) + 0.5 * (Q(c + 1) - Q(c));
-    const double *p = zm.ppmc + 12 * (c - 1);
-    double ffip1 = Q(c + 1) - Q(c), ffip2 = Q(c + 2) - Q(c + 1), ffim1 = Q(c) - Q(c - 1);
-    double sl = p[0] * (p[1] * ffip1 + p[2] * ffim1);
-    double slp1 = p[3] * (p[4] * ffip2 + p[5] * ffip1);
-    return Q(c) + p[6] * ffip1 + p[7] * (p[8] * ffip1 - p[9] * slp1 + p[10] * sl);
-}
-
-// Flux_r/Flux_l of level c in 1..nz-1, advsz_ppm (advq_ppm.f90:326-409)
-template <class QF, class WF>
-__device__ __forceinline__ PPMRec ppm_zcell(int c, int nz, const ZMetrics &zm, const SchemeParams &sp,
-                                            double bc51, double bc61, QF Q, WF W)
-{
-    double dt0 = sp.dt0;
-    double dz1c = zm.dz1[c - 1];
-    double mup = fabs(W(c + 1)) * dt0 * dz1c;
-    double muc = fabs(W(c)) * dt0 * dz1c;
-    double xx = Q(c), xp = Q(c + 1);
-    double ffip1 = xp - xx;
-    if (c == 1) {
-        double ffip2 = Q(3) - xp;
-        double ffim1 = bc51 * (Q(nz - 4) - Q(nz - 5));
-        double ffim2 = bc51 * (Q(nz - 5) - Q(nz - 6));
-        double xmin = xx - 0.5 * ffip1;
-        double xplus = xx + 0.5 * ffip1;
-        return ppm_cell(sp.ppm_limiter, xx, xp, xp, xplus, xmin, ffip1, ffip2, ffim1, ffim2, mup, muc);
-    }
-    double xm = Q(c - 1);
-    double xmin = ppm_zxplus(c - 1, zm, Q);
-    if (c == 2) {
-        double ffip2 = Q(4) - xp;
-        double ffim1 = xx - xm;
-        double ffim2 = bc51 * (Q(nz - 4) - Q(nz - 5));
-        double xplus = xx + 0.5 * ffip1;
-        return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim2, mup, muc);
-    }
-    double ffim1 = xx - xm, ffim2 = xm - Q(c - 2);
-    if (c == nz - 1) {
-        double ffip2 = bc61 * (Q(6) - Q(5)) + (1.0 - bc61) * ffip1;
-        double xplus = xx + 0.5 * ffip1;
-        return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim2, mup, muc);
-    }
-    double ffip2 = Q(c + 2) - xp;
-    double xplus = ppm_zxplus(c, zm, Q);
-    return ppm_cell(sp.ppm_limiter, xx, xp, xm, xplus, xmin, ffip1, ffip2, ffim1, ffim2, mup, muc);
-}
-
-// Flux_l of the top level (advq_ppm.f90:411-414)
-template <class QF, class WF>
-__device__ __forceinline__ double ppm_ztop_fl(int nz, const ZMetrics &zm, const SchemeParams &sp, QF Q, WF W)
-{
-    double muc = fabs(W(nz)) * sp.dt0 * zm.dz1[nz - 1];
-    double ffim1 = Q(nz) - Q(nz - 1);
-    return Q(nz) + 0.5 * ffim1 * (1.0 - muc);
-}
-
-// ---------------------------------------------------------------------------
-// z contributions: the tendency loop of advs z_* (face differences, adv
-// term, nnf closures), same for all three schemes
-// ---------------------------------------------------------------------------
-
-template <class FF, class QF, class WF>
-__device__ __forceinline__ double z_assemble(int k, int nz, bool adv, int bc5, int bc6, const ZMetrics &zm,
-                                             FF face, QF Q, WF W)
-{
-    const double *dz1w = zm.dz1w;
-    if (k >= 2 && k <= nz - 1) {
-        double t = (face(k) - face(k - 1)) * dz1w[k - 1];
-        if (adv) t = t - Q(k) * (W(k + 1) - W(k)) * dz1w[k - 1];
-        return t;
-    }
-    double t = 0.0;
-    if (k == 1 && bc5 == 1) {
-        t = t + (face(1) - 0.0) * dz1w[0];
-        if (adv) t = t - Q(1) * (W(2) - 0.0) * dz1w[0];
-    }
-    if (k == nz && bc6 == 1) {
-        t = t + (0.0 - face(nz - 1)) * dz1w[nz - 1];
-        if (adv) t = t - Q(nz) * (0.0 - W(nz)) * dz1w[nz - 1];
-    }
-    return t;
+    if (c <= 2 || c == nz - 1) return x + 0.5 * d;
+    const double *p = ppmc + 12 * (c - 1);
+    const double sl = p[0] * (p[1] * d + p[2] * dm);
+    const double slp1 = p[3] * (p[4] * dp + p[5] * d);
+    return x + p[6] * d + p[7] * (p[8] * d - p[9] * slp1 + p[10] * sl);
 }
 
 }  // namespace mimadv

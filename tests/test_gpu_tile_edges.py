@@ -37,8 +37,8 @@ def test_momentum_tile_edges(cuda, dims, bc, ntime, lavisc):
             assert np.array_equal(outs[c].cpu().numpy(), ref[c]), f"component {c}"
 
 
-@pytest.mark.parametrize("scheme", ["weno", "weno5", "muscl"])
-@pytest.mark.parametrize("dims", [(139, 117, 75), (6, 6, 8), (33, 9, 8), (300, 0, 41), (1500, 0, 301)])
+@pytest.mark.parametrize("scheme", ["weno", "weno5", "muscl", "ppm"])
+@pytest.mark.parametrize("dims", [(139, 117, 75), (6, 6, 8), (33, 9, 8), (15, 17, 33), (300, 0, 41), (1500, 0, 301)])
 def test_scalar_chunk_lengths(cuda, scheme, dims):
     """Grids for which the dispatch takes one level per item, a few (with a
     shorter last chunk) and several; the other tests' grids take one."""
@@ -87,3 +87,22 @@ def test_scratch_contents_do_not_matter(cuda, what, two_d):
         call(a, torch.full_like(field, float("nan")))
         for x, y in zip(call(a, field), call(b, field)):
             assert np.isfinite(x).all() and np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("dirs", [1, 2, 4, 5, 7])
+@pytest.mark.parametrize("bc", ["nnf", "ope", "per"])
+@pytest.mark.parametrize("side", ["per", "ope"])
+def test_ppm_directions_and_boundaries(cuda, dirs, bc, side):
+    """Every direction subset, vertical boundary code and side code (the
+    non-periodic sides take another flux at the last interior cell), flux and
+    advective form, on a grid of several tiles and chunks."""
+    print(f"case ppm dirs={dirs} {bc} {side}", flush=True)
+    g, u, v, w, q = case3d(47, 19, 75, bcl=(side,) * 4 + (bc, bc))
+    for adv in (False, True):
+        ref = np.full(g.shape, 0.25)
+        Oracle(g, scal_adv="ppm").scalar_tendency(2.0, u, v, w, q, ref, adv, dirs)
+        with Advection(g, scal_adv="ppm") as a:
+            du, dv, dw, dq, dx = _dev(cuda, u, v, w, q, np.full(g.shape, 0.25))
+            a.scalar_tendency(2.0, du, dv, dw, [dq], [dx], [adv], dirs=dirs)
+            a.stream_sync()
+            assert np.array_equal(dx.cpu().numpy(), ref)
