@@ -92,6 +92,61 @@ __device__ __forceinline__ double muscl_upwind(double uu, double fl, double fr)
     return 0.5 * uu * (fl * (1.0 + sgn1(uu)) + fr * (1.0 - sgn1(uu)));
 }
 
+// |p| < |s| / lt (lt > 0) with the outcome of the rounded quotient: p lt and s
+// differ by more than 2^-50 of s, or the division decides
+__device__ __forceinline__ bool below_ratio(double p, double s, double lt)
+{
+    const double t = fma(-lt, fabs(p), fabs(s));
+    bool r = t > 0.0;
+    if (__builtin_expect(fabs(t) <= fabs(s) * 0x1p-50, 0)) r = fabs(p) < fabs(s) / lt;
+    return r;
+}
+
+// Face flux from the two cell values, the slopes at the face and at its
+// neighbours and the gate of the limiter.  `term(x)` scales a slope product to
+// a value difference (x d in x and y, x / dz1w in z).
+//
+// The reference forms both sides' values and multiplies the off-side one by an
+// exact zero, so with finite slopes the upwind side alone gives the flux (a
+// zero may differ in sign); this halves the work and leaves one division of
+// four (197 -> 168 us per launch at 256x256x128, 'MC').  Slopes that are not finite, or so large that a product may
+// overflow, take the reference's sum, in which an infinite off side gives NaN.
+template <class TF>
+__device__ __forceinline__ double muscl_flux(const SchemeParams &sp, double uu, double xx, double xp, double slope_p,
+                                             double slope_p2, double slope_m, bool limited, TF term)
+{
+    const double lt = sp.lim_tol;
+    if (__builtin_expect(!(fabs(slope_m) + fabs(slope_p2) < 0x1p400 && fabs(slope_p) < 0x1p400), 0)) {
+        double phir, phil, fl, fr;
+        if (limited) {
+            muscl_limiter(sp.muscl_limiter, lt, xx, slope_p, slope_p2, slope_m, phir, phil);
+            fr = xp - term(0.5 * phir * slope_p2);
+            fl = xx + term(0.5 * phil * slope_m);
+        } else {
+            fr = xp - term(0.5 * slope_p);
+            fl = xx + term(0.5 * slope_p);
+        }
+        return muscl_upwind(uu, fl, fr);
+    }
+    const bool pos = !signbit(uu);
+    const double so = pos ? slope_m : slope_p2, base = pos ? xx : xp;
+    double v = 0.5 * slope_p;
+    if (limited) {
+        double r = 1.0;
+        if (fabs(so) > lt * fabs(xx) && below_ratio(slope_p, so, lt)) r = quotient(slope_p, so);
+        double phi;
+        switch (sp.muscl_limiter) {
+        case 2: phi = (r + fabs(r)) / (1.0 + fabs(r)); break;                                 // VL
+        case 1: phi = fmax(0.0, fmin(fmin(2.0 * r, 0.5 * (r + 1.0)), 2.0)); break;            // MC
+        case 0: phi = fmax(0.0, fmin(1.0, r)); break;                                         // minmod
+        default: phi = 0.5 * (r + 1.0); break;                                                // Fromm
+        }
+        v = 0.5 * phi * so;
+    }
+    v = term(v);
+    return uu * (pos ? base + v : base - v);
+}
+
 // face flux i+1/2, x/y (advq_muscl.f90:81-100)
 template <class QF, class UF>
 __device__ __forceinline__ double muscl_hface(int i, double d, double d1, const SchemeParams &sp, QF Q, UF U)
@@ -102,18 +157,9 @@ __device__ __forceinline__ double muscl_hface(int i, double d, double d1, const 
     double slope_p = (xp - xx) * d1;
     double slope_p2 = (Q(i + 2) - xp) * d1;
     double slope_m = (xx - Q(i - 1)) * d1;
-    double lt = sp.lim_tol;
-    double fl, fr;
-    if (d * fabs(slope_m) > lt * fabs(xx) + eps || d * fabs(slope_p2) > lt * fabs(xx) + eps) {
-        double phir, phil;
-        muscl_limiter(sp.muscl_limiter, lt, xx, slope_p, slope_p2, slope_m, phir, phil);
-        fr = xp - 0.5 * phir * slope_p2 * d;
-        fl = xx + 0.5 * phil * slope_m * d;
-    } else {
-        fr = xp - 0.5 * slope_p * d;
-        fl = xx + 0.5 * slope_p * d;
-    }
-    return muscl_upwind(uu, fl, fr);
+    const double gate = sp.lim_tol * fabs(xx) + eps;
+    const bool limited = (d * fabs(slope_m) > gate) | (d * fabs(slope_p2) > gate);
+    return muscl_flux(sp, uu, xx, xp, slope_p, slope_p2, slope_m, limited, [&](double x) { return x * d; });
 }
 
 // z face flux k+1/2 (advsz_muscl, advq_muscl.f90:245-302)
@@ -122,46 +168,28 @@ __device__ __forceinline__ double muscl_zface(int f, int nz, const ZMetrics &zm,
                                               double bc51, double bc61, QF Q, WF W)
 {
     const double eps = 1.e-18;
-    double lt = sp.lim_tol, dz = zm.dz;
-    const double *dz1 = zm.dz1, *dz1w = zm.dz1w, *fdz0 = zm.fdz0;
-    double ww = W(f + 1);
-    double slope_p, slope_p2, slope_m, phir, phil, fl, fr;
-    double m = dz1w[f - 1];
-    if (f == 1) {
-        slope_p = (Q(2) - Q(1)) * dz1[0];
-        slope_p2 = (Q(3) - Q(2)) * dz1[1];
-        slope_m = bc51 * (Q(nz - 4) - Q(nz - 5)) * dz1[nz - 6] + (1.0 - bc51) * slope_p;
-        if (fdz0[1] * dz * fabs(slope_p2) > lt * fabs(Q(1)) + eps) {
-            muscl_limiter(sp.muscl_limiter, lt, Q(1), slope_p, slope_p2, slope_m, phir, phil);
-            fl = Q(1) + 0.5 * phil * slope_m / m;
-            fr = Q(2) - 0.5 * phir * slope_p2 / m;
-        } else {
-            fl = Q(1) + 0.5 * slope_p / m;
-            fr = Q(2) - 0.5 * slope_p / m;
-        }
-        return muscl_upwind(ww, fl, fr);
-    }
-    double xk = Q(f), xp = Q(f + 1);
-    slope_p = (xp - xk) * dz1[f - 1];
-    slope_m = (xk - Q(f - 1)) * dz1[f - 2];
+    double dz = zm.dz;
+    const double *dz1 = zm.dz1, *fdz0 = zm.fdz0;
+    const LevelDiv m(zm.dz1w[f - 1]);
+    const double xx = Q(f), xp = Q(f + 1), gate = sp.lim_tol * fabs(xx) + eps;
+    const double slope_p = (xp - xx) * dz1[f - 1];
+    double slope_p2, slope_m;
     bool limited;
-    if (f == nz - 1) {
+    if (f == 1) {
+        slope_p2 = (Q(3) - xp) * dz1[1];
+        slope_m = bc51 * (Q(nz - 4) - Q(nz - 5)) * dz1[nz - 6] + (1.0 - bc51) * slope_p;
+        limited = fdz0[1] * dz * fabs(slope_p2) > gate;
+    } else if (f == nz - 1) {
+        slope_m = (xx - Q(f - 1)) * dz1[f - 2];
         slope_p2 = bc61 * (Q(6) - Q(5)) * dz1[4] + (1.0 - bc61) * slope_p;
-        limited = fdz0[f - 2] * dz * fabs(slope_m) > lt * fabs(xk) + eps;
+        limited = fdz0[f - 2] * dz * fabs(slope_m) > gate;
     } else {
+        slope_m = (xx - Q(f - 1)) * dz1[f - 2];
         slope_p2 = (Q(f + 2) - xp) * dz1[f];
-        limited = fdz0[f - 2] * dz * fabs(slope_m) > lt * fabs(xk) + eps ||
-                  fdz0[f] * dz * fabs(slope_p2) > lt * fabs(xk) + eps;
+        limited = (fdz0[f - 2] * dz * fabs(slope_m) > gate) | (fdz0[f] * dz * fabs(slope_p2) > gate);
     }
-    if (limited) {
-        muscl_limiter(sp.muscl_limiter, lt, xk, slope_p, slope_p2, slope_m, phir, phil);
-        fr = xp - 0.5 * phir * slope_p2 / m;
-        fl = xk + 0.5 * phil * slope_m / m;
-    } else {
-        fr = xp - 0.5 * slope_p / m;
-        fl = xk + 0.5 * slope_p / m;
-    }
-    return muscl_upwind(ww, fl, fr);
+    return muscl_flux(sp, W(f + 1), xx, xp, slope_p, slope_p2, slope_m, limited,
+                      [&](double x) { return m.div(x); });
 }
 
 // ---------------------------------------------------------------------------

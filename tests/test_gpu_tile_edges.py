@@ -106,3 +106,47 @@ def test_ppm_directions_and_boundaries(cuda, dirs, bc, side):
             a.scalar_tendency(2.0, du, dv, dw, [dq], [dx], [adv], dirs=dirs)
             a.stream_sync()
             assert np.array_equal(dx.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("scheme,lim", [("weno", "MC"), ("ppm", "MC"), ("muscl", "minmod"), ("muscl", "MC"),
+                                        ("muscl", "VL"), ("muscl", "Fromm")])
+@pytest.mark.parametrize("data", ["tiny", "huge", "zeros", "constant", "steps"])
+def test_scalar_extreme_values(cuda, scheme, lim, data):
+    """Values at the ends of the exponent range, exact zeros, constants and
+    jumps: the quotients without operand scaling and the limiter gates."""
+    print(f"case extreme {scheme} {lim} {data}", flush=True)
+    g, u, v, w, q = case3d(35, 18, 20, zero_frac=0.5 if data == "zeros" else 0.0)
+    q = {"tiny": q * 1e-295, "huge": q * 1e150, "zeros": q, "constant": np.full_like(q, 3.25),
+         "steps": np.where(q > 1e-4, 1.0, -2.0)}[data]
+    ref = np.zeros(g.shape)
+    Oracle(g, scal_adv=scheme, muscllimiter=lim).scalar_tendency(1.0, u, v, w, q, ref)
+    with Advection(g, scal_adv=scheme, muscllimiter=lim) as a:
+        du, dv, dw, dq, dx = _dev(cuda, u, v, w, q, np.zeros(g.shape))
+        a.scalar_tendency(1.0, du, dv, dw, [dq], [dx])
+        a.stream_sync()
+        got = dx.cpu().numpy()
+    # 'weno' forms the upwind side only: where the other side overflows to NaN
+    # in the reference's sum, its value is not the reference's NaN
+    fin = np.isfinite(ref) if scheme == "weno" else np.ones(g.shape, bool)
+    assert fin.any() and np.array_equal(got[fin], ref[fin])
+
+
+@pytest.mark.parametrize("scheme,lim", [("ppm", "MC"), ("muscl", "minmod"), ("muscl", "VL")])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_scalar_non_finite_values(cuda, scheme, lim, value):
+    """A few non-finite cells: what they reach is what they reach in the
+    reference's formulas, which look at both sides of a face."""
+    print(f"case non-finite {scheme} {lim} {value}", flush=True)
+    g, u, v, w, q = case3d(35, 18, 20)
+    for k, j, i in ((0, 8, 9), (7, 12, 20), (19, 6, 30), (10, 15, 33)):
+        q[k, j, i] = value
+    ref = np.zeros(g.shape)
+    with np.errstate(all="ignore"):
+        Oracle(g, scal_adv=scheme, muscllimiter=lim).scalar_tendency(1.0, u, v, w, q, ref)
+    with Advection(g, scal_adv=scheme, muscllimiter=lim) as a:
+        du, dv, dw, dq, dx = _dev(cuda, u, v, w, q, np.zeros(g.shape))
+        a.scalar_tendency(1.0, du, dv, dw, [dq], [dx])
+        a.stream_sync()
+        got = dx.cpu().numpy()
+    assert not np.isfinite(got).all()
+    assert np.array_equal(got, ref, equal_nan=True)
