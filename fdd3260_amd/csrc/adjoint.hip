@@ -238,6 +238,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
     __shared__ unsigned slots[(QS + LS + FS) * NT];
 
     const int nx = A.nx, ny = A.ny, nz = A.nz, mx = nx - 5, my = ny - 5;
+    const auto dz1w = table(A.dz1w);
     const size_t plane = (size_t)nx * ny;
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
     const int nchunk = (nz + A.kchunk - 1) / A.kchunk;
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
             }
             // z face k+1/2 (velocity w(k+1)); no flux through floor and lid
             if (k <= nz - 1) {
-                const double Fb = A.ls * (qbw[ZL + 1] * A.dz1w[k] - qbw[ZL] * A.dz1w[k - 1]);
+                const double Fb = A.ls * (qbw[ZL + 1] * dz1w[k] - qbw[ZL] * dz1w[k - 1]);
                 const bool upos = !(wz < 0.0);
                 double R;
                 if (S5 && wz > 0.0 && k >= 3 && k <= nz - 2) {

@@ -187,7 +187,7 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
             if (sl.t_off[s] >= 0) tv[s] = load_at(qk, tb[s]);
         if (need_q0 && valid) q0v = load_at(q0 + kb, colb);
         zn = load_at(q + lev(k + H), colb);
-        d1v = A.dz1w[k - 1];
+        d1v = table(A.dz1w)[k - 1];
     };
     fetch(k0);
 #pragma unroll 1

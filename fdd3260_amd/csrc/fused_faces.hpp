@@ -4,6 +4,7 @@
 // index wrap.  Shared by the single-grid and multi-domain batched kernels.
 #pragma once
 #include "fused.hpp"
+#include "metric.hpp"
 
 namespace mimadv {
 namespace faces {
@@ -177,8 +178,8 @@ __device__ __forceinline__ T muscl_zface(int f, int nz, T a, T b, T c, T d, T ww
     const T eps = T(1e-18);
     const int lim = A.muscl_limiter;
     const T lt = T(A.lim_tol), rlt = T(A.lim_tol_inv), dz = T(A.dz);
-    const double *dz1 = A.dz1, *fdz0 = A.fdz0;
-    const T m = T(A.dzw[f - 1]);  // 1/dz1w(f)
+    const auto dz1 = table(A.dz1), fdz0 = table(A.fdz0);
+    const T m = T(table(A.dzw)[f - 1]);  // 1/dz1w(f)
     const T sp = (c - b) * T(dz1[f - 1]);
     T sm, sp2;
     bool limited;

@@ -94,7 +94,7 @@ __device__ __forceinline__ float cross_line(int i, float d1, float d3, const Mom
 // W(kk, o) the vertical velocity at level kk and transverse offset o;
 // m2k the level of dz1w on the k = 2 line (1 for u, 2 for v)
 template <class MF, class WF>
-__device__ __forceinline__ float cross_z(int k, int nz, const float *mz, int m2k, const MomF &c, MF M, WF W)
+__device__ __forceinline__ float cross_z(int k, int nz, Table<float> mz, int m2k, const MomF &c, MF M, WF W)
 {
     auto Zc = [&](int kk, int n) { return mz[MOMZ_N * (kk - 1) + n]; };
     auto flux = [&](int kk) -> float {
@@ -140,7 +140,7 @@ __device__ __forceinline__ float w_line(int i, int k, int nz, float d1, float d3
 
 // advwz_fd with 'nnf' floor and lid (windadv.f90:1058-1127)
 template <class MF, class TF>
-__device__ __forceinline__ float w_z(int k, int nz, const float *mz, const MomF &c, MF M, TF T)
+__device__ __forceinline__ float w_z(int k, int nz, Table<float> mz, const MomF &c, MF M, TF T)
 {
     auto Zc = [&](int kk, int n) { return mz[MOMZ_N * (kk - 1) + n]; };
     auto flux = [&](int kk) -> float {
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
     const int nchunk = (nz + kchunk - 1) / kchunk;
     const float *src[6] = {a.m[0], a.m[1], a.m[2], a.ut, a.vt, a.wt};
-    const float *mz = g.zm.momz;
+    const auto mz = table(g.zm.momz);
 
     if (const int wi = blockIdx.x; wi < nwork) {
         // Work order: level chunk outermost, tiles x-fastest within it.  The

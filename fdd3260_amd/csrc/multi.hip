@@ -118,7 +118,7 @@ __device__ __forceinline__ void march_multi(const FusedArgs &A, const Geom &G, c
             if (sl.t_off[s] >= 0) tv[s] = load_at(qk, tb[s]);
         if (need_q0 && valid) q0v = load_at(q0 + kb, colb);
         zn = load_at(q + lev(k + H), colb);
-        d1v = A.dz1w[k - 1];
+        d1v = table(A.dz1w)[k - 1];
     };
     const int ex = ty * (G.TX + 1) + tx, ey = G.NXF + ty * G.TX + tx;
     fetch(k0);

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                zdir = (a.dirmask & 4) != 0;
     const int bc5 = g.bcl[4], bc6 = g.bcl[5];
     const double bc51 = bc5 == 0 ? 1.0 : 0.0, bc61 = bc6 == 0 ? 1.0 : 0.0;
-    const double *__restrict__ dz1w = g.zm.dz1w, *__restrict__ dz1 = g.zm.dz1, *__restrict__ ppmc = g.zm.ppmc;
+    const auto dz1w = table(g.zm.dz1w), dz1 = table(g.zm.dz1), ppmc = table(g.zm.ppmc);
     const bool accum = a.epi == EPI_ACCUM, heun = a.epi == EPI_HEUN, so = a.epi == EPI_SO;
     const bool need_tend = heun && a.b_lm != 0.0;
     // the array the epilogue starts from: the tendency or the step-start state

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fp64_div.hpp"
+#include "metric.hpp"
 #include "weno_ratio.hpp"
 
 namespace mimadv {
@@ -169,8 +170,8 @@ __device__ __forceinline__ double muscl_zface(int f, int nz, const ZMetrics &zm,
 {
     const double eps = 1.e-18;
     double dz = zm.dz;
-    const double *dz1 = zm.dz1, *fdz0 = zm.fdz0;
-    const LevelDiv m(zm.dz1w[f - 1]);
+    const auto dz1 = table(zm.dz1), fdz0 = table(zm.fdz0);
+    const LevelDiv m(table(zm.dz1w)[f - 1]);
     const double xx = Q(f), xp = Q(f + 1), gate = sp.lim_tol * fabs(xx) + eps;
     const double slope_p = (xp - xx) * dz1[f - 1];
     double slope_p2, slope_m;
@@ -250,7 +251,7 @@ template <class QF>
 __device__ __forceinline__ void z_slopes(int f, int nz, const ZMetrics &zm, double bc51, double bc61, QF Q,
                                          double ffip1, double &ffip2, double &ffim1)
 {
-    const double *dz1 = zm.dz1;
+    const auto dz1 = table(zm.dz1);
     if (f == 1) {
         ffip2 = (Q(3) - Q(2)) * dz1[1];
         ffim1 = bc51 * (Q(nz - 4) - Q(nz - 5)) * dz1[nz - 6] + (1.0 - bc51) * ffip1;
@@ -269,10 +270,10 @@ __device__ __forceinline__ double quick_zface(int f, int nz, const ZMetrics &zm,
                                               double bc51, double bc61, QF Q, WF W)
 {
     double xx = Q(f), ww = W(f + 1), xp = Q(f + 1);
-    double ffip1 = (xp - xx) * zm.dz1[f - 1];
+    double ffip1 = (xp - xx) * table(zm.dz1)[f - 1];
     double ffip2, ffim1;
     z_slopes(f, nz, zm, bc51, bc61, Q, ffip1, ffip2, ffim1);
-    const double m = zm.dz1w[f - 1];
+    const double m = table(zm.dz1w)[f - 1];
     double phil, phir, fl, fr;
     if constexpr (NL) {
         const double cc = 1.0 / 4.0;
@@ -347,9 +348,9 @@ __device__ __forceinline__ double lw_zface(int f, int nz, const ZMetrics &zm, co
 {
     const double eps = 1.e-18;
     double xx = Q(f), ww = W(f + 1), xp = Q(f + 1);
-    double mu = fabs(ww) * sp.dt0 * zm.dz1[f - 1];
-    double ffip1 = (xp - xx) * zm.dz1[f - 1];
-    const double m = zm.dz1w[f - 1];
+    double mu = fabs(ww) * sp.dt0 * table(zm.dz1)[f - 1];
+    double ffip1 = (xp - xx) * table(zm.dz1)[f - 1];
+    const double m = table(zm.dz1w)[f - 1];
     double fl, fr;
     if constexpr (NL) {
         fl = xx + 0.5 * ffip1 * (1.0 - mu) / m;
@@ -485,10 +486,10 @@ __device__ __forceinline__ double ppm_faceflux(double fr, double fl, double uf)
 //  [6] delta/(delta+dp1)       [7] 1/(dm1+delta+dp1+dp2)
 //  [8] 2dp1*delta/(delta+dp1)*((dm1+delta)/(2delta+dp1)-(dp2+dp1)/(2dp1+delta))
 //  [9] delta*(dm1+delta)/(2delta+dp1)   [10] dp1*(dp1+dp2)/(2dp1+delta)
-__device__ __forceinline__ double ppm_zxplus(int c, int nz, const double *ppmc, double x, double dm, double d, double dp)
+__device__ __forceinline__ double ppm_zxplus(int c, int nz, Table<double> ppmc, double x, double dm, double d, double dp)
 {
     if (c <= 2 || c == nz - 1) return x + 0.5 * d;
-    const double *p = ppmc + 12 * (c - 1);
+    const auto p = ppmc + 12 * (c - 1);
     const double sl = p[0] * (p[1] * d + p[2] * dm);
     const double slp1 = p[3] * (p[4] * dp + p[5] * d);
     return x + p[6] * d + p[7] * (p[8] * d - p[9] * slp1 + p[10] * sl);

@@ -240,7 +240,7 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
     const bool adv = a.adv != 0;
     const int bc5 = g.bcl[4], bc6 = g.bcl[5];
     const double bc51 = bc5 == 0 ? 1.0 : 0.0, bc61 = bc6 == 0 ? 1.0 : 0.0;  // periodic floor, lid
-    const double *__restrict__ dz1w = g.zm.dz1w;
+    const auto dz1w = table(g.zm.dz1w);
     const bool zdir = (a.dirmask & 4) != 0;
     const bool accum = a.epi == EPI_ACCUM, heun = a.epi == EPI_HEUN, so = a.epi == EPI_SO;
     const bool need_tend = heun && a.b_lm != 0.0, need_q0 = heun || so;
