@@ -2,7 +2,7 @@
 //
 // A batch of unequal subdomains (each with its own grid, metrics, FP32
 // velocity, dt, scheme and set of FP32 fields) is advanced by one
-// persistent launch per Shu-Osher stage.  The subdomains' work items (a
+// launch per Shu-Osher stage.  The subdomains' work items (a
 // tile of columns and a chunk of levels) are numbered consecutively; a
 // workgroup finds its subdomain by a binary search of the first work id of
 // every subdomain, reads that subdomain's argument block from a device
@@ -191,99 +191,96 @@ __device__ __forceinline__ void march_multi(const FusedArgs &A, const Geom &G, c
 // Six-level work items take 25 KB of LDS; the register budget is held to
 // five waves per SIMD (96 VGPRs; three values are reloaded per level).
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5, 8))) void multi_kernel(
-    const FusedArgs *__restrict__ table, int ndom, int nwork)
+    const FusedArgs *__restrict__ table, int ndom)
 {
     __shared__ float tile_lds[TILE_MAX];
     __shared__ float face_lds[FS * NT];
     __shared__ float vel_lds[KC_MAX * NV_MAX];
     const int tid = threadIdx.x;
-    for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
-        // subdomain of this work id: last d with work_begin <= wi
-        int lo = 0, hi = ndom - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (table[mid].work_begin <= wi) lo = mid;
-            else hi = mid - 1;
+    const int wi = blockIdx.x;
+    // subdomain of this work id: last d with work_begin <= wi
+    int lo = 0, hi = ndom - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (table[mid].work_begin <= wi) lo = mid;
+        else hi = mid - 1;
+    }
+    // a private copy of the argument block: its scalars stay in registers
+    // instead of being reloaded after every store (the table is global
+    // memory); the field pointers are read from the table once per field
+    const FusedArgs A = table[lo];
+    Geom G;
+    G.set(A.tile_x, A.tile_y, A.scheme == 3 ? 3 : 2);
+    const int local = wi - A.work_begin;
+    const int tiles = A.ntx * A.nty;
+    const int chunk = local / tiles, t = local - chunk * tiles;
+    const int i0 = 4 + (t % A.ntx) * G.TX, j0 = 4 + (t / A.ntx) * G.TY;
+    const int k0 = 1 + chunk * A.kchunk, nk = min(A.kchunk, A.nz - k0 + 1);
+    const int tx = tid % G.TX, ty = tid / G.TX;
+    const int i = i0 + tx, j = j0 + ty;
+    const bool valid = i <= A.nx - 2 && j <= A.ny - 2;
+    const int col = (wrap(i, A.nx, A.mx) - 1) + A.nx * (wrap(j, A.ny, A.my) - 1);
+    SlotsR sl;
+    sl.init(G, tid, i0, j0, A);
+    // the chunk's face velocities and column w(k+1), read once for every
+    // field: each staging slot's source array and plane offset are fixed
+    // for the item, and all the chunk's loads are in flight together before
+    // they go to LDS
+    {
+        constexpr int VS = (NV_MAX + NT - 1) / NT;
+        const int nx = A.nx, ny = A.ny;
+        const size_t plane = (size_t)nx * ny;
+        const float *vp[VS];
+        int voff[VS];
+        bool vw[VS];
+#pragma unroll
+        for (int s = 0; s < VS; ++s) {
+            const int e = tid + s * NT;
+            vp[s] = A.u;
+            voff[s] = -1;
+            vw[s] = false;
+            if (e < G.NXF) {
+                const int r = e / (G.TX + 1), fl = e - r * (G.TX + 1);
+                voff[s] = (wrap(i0 + fl, nx, A.mx) - 1) + nx * (wrap(j0 + r, ny, A.my) - 1);
+            } else if (e < G.NF) {
+                const int e2 = e - G.NXF, fr = e2 / G.TX, c = e2 - fr * G.TX;
+                vp[s] = A.v;
+                voff[s] = (wrap(i0 + c, nx, A.mx) - 1) + nx * (wrap(j0 + fr, ny, A.my) - 1);
+            } else if (e < G.NV) {
+                const int c = e - G.NF, cx = c % G.TX, cy = c / G.TX;
+                vp[s] = A.w;  // w(k+1) at level k
+                voff[s] = (wrap(i0 + cx, nx, A.mx) - 1) + nx * (wrap(j0 + cy, ny, A.my) - 1);
+                vw[s] = true;
+            }
         }
-        // a private copy of the argument block: its scalars stay in registers
-        // instead of being reloaded after every store (the table is global
-        // memory); the field pointers are read from the table once per field
-        const FusedArgs A = table[lo];
-        Geom G;
-        G.set(A.tile_x, A.tile_y, A.scheme == 3 ? 3 : 2);
-        const int local = wi - A.work_begin;
-        const int tiles = A.ntx * A.nty;
-        const int chunk = local / tiles, t = local - chunk * tiles;
-        const int i0 = 4 + (t % A.ntx) * G.TX, j0 = 4 + (t / A.ntx) * G.TY;
-        const int k0 = 1 + chunk * A.kchunk, nk = min(A.kchunk, A.nz - k0 + 1);
-        const int tx = tid % G.TX, ty = tid / G.TX;
-        const int i = i0 + tx, j = j0 + ty;
-        const bool valid = i <= A.nx - 2 && j <= A.ny - 2;
-        const int col = (wrap(i, A.nx, A.mx) - 1) + A.nx * (wrap(j, A.ny, A.my) - 1);
-        SlotsR sl;
-        sl.init(G, tid, i0, j0, A);
-        // the chunk's face velocities and column w(k+1), read once for every
-        // field: each staging slot's source array and plane offset are fixed
-        // for the item, and all the chunk's loads are in flight together
-        // (issued before the barrier that waits for the previous item's
-        // fields) before they go to LDS
-        {
-            constexpr int VS = (NV_MAX + NT - 1) / NT;
-            const int nx = A.nx, ny = A.ny;
-            const size_t plane = (size_t)nx * ny;
-            const float *vp[VS];
-            int voff[VS];
-            bool vw[VS];
+        float vb[KC_MAX][VS];
+#pragma unroll
+        for (int kk = 0; kk < KC_MAX; ++kk) {
+            const int k = k0 + kk;
 #pragma unroll
             for (int s = 0; s < VS; ++s) {
-                const int e = tid + s * NT;
-                vp[s] = A.u;
-                voff[s] = -1;
-                vw[s] = false;
-                if (e < G.NXF) {
-                    const int r = e / (G.TX + 1), fl = e - r * (G.TX + 1);
-                    voff[s] = (wrap(i0 + fl, nx, A.mx) - 1) + nx * (wrap(j0 + r, ny, A.my) - 1);
-                } else if (e < G.NF) {
-                    const int e2 = e - G.NXF, fr = e2 / G.TX, c = e2 - fr * G.TX;
-                    vp[s] = A.v;
-                    voff[s] = (wrap(i0 + c, nx, A.mx) - 1) + nx * (wrap(j0 + fr, ny, A.my) - 1);
-                } else if (e < G.NV) {
-                    const int c = e - G.NF, cx = c % G.TX, cy = c / G.TX;
-                    vp[s] = A.w;  // w(k+1) at level k
-                    voff[s] = (wrap(i0 + cx, nx, A.mx) - 1) + nx * (wrap(j0 + cy, ny, A.my) - 1);
-                    vw[s] = true;
-                }
+                vb[kk][s] = 0.0f;
+                if (kk < nk && voff[s] >= 0 && (!vw[s] || k < A.nz))
+                    vb[kk][s] = vp[s][(size_t)(vw[s] ? k : k - 1) * plane + (size_t)voff[s]];
             }
-            float vb[KC_MAX][VS];
-#pragma unroll
-            for (int kk = 0; kk < KC_MAX; ++kk) {
-                const int k = k0 + kk;
-#pragma unroll
-                for (int s = 0; s < VS; ++s) {
-                    vb[kk][s] = 0.0f;
-                    if (kk < nk && voff[s] >= 0 && (!vw[s] || k < A.nz))
-                        vb[kk][s] = vp[s][(size_t)(vw[s] ? k : k - 1) * plane + (size_t)voff[s]];
-                }
-            }
-            __syncthreads();  // the previous item's fields are done with vel_lds
-#pragma unroll
-            for (int kk = 0; kk < KC_MAX; ++kk)
-#pragma unroll
-                for (int s = 0; s < VS; ++s)
-                    if (kk < nk && tid + s * NT < G.NV) vel_lds[kk * G.NV + tid + s * NT] = vb[kk][s];
-            __syncthreads();
         }
+#pragma unroll
+        for (int kk = 0; kk < KC_MAX; ++kk)
+#pragma unroll
+            for (int s = 0; s < VS; ++s)
+                if (kk < nk && tid + s * NT < G.NV) vel_lds[kk * G.NV + tid + s * NT] = vb[kk][s];
+        __syncthreads();
+    }
 #pragma unroll 1
-        for (int f = 0; f < A.n32_active; ++f) {
-            const float *qf = table[lo].q32[f], *q0f = table[lo].q0_32[f];
-            float *of = table[lo].out32[f];
-            if (A.scheme == 0)
-                march_multi<0>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
-            else if (A.scheme == 3)
-                march_multi<3>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
-            else
-                march_multi<2>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
-        }
+    for (int f = 0; f < A.n32_active; ++f) {
+        const float *qf = table[lo].q32[f], *q0f = table[lo].q0_32[f];
+        float *of = table[lo].out32[f];
+        if (A.scheme == 0)
+            march_multi<0>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
+        else if (A.scheme == 3)
+            march_multi<3>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
+        else
+            march_multi<2>(A, G, qf, q0f, of, tile_lds, face_lds, vel_lds, k0, nk, i0, j0, tid, tx, ty, valid, col, sl);
     }
 }
 
@@ -306,14 +303,12 @@ void multi_prepare(FusedArgs &A, int work_begin)
 hipError_t launch_multi(const FusedArgs *d_table, int ndom, int nwork, hipStream_t s)
 {
     if (ndom <= 0 || nwork <= 0) return hipSuccess;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
-        ncu = 256;
-    int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, multi_kernel, NT, 0) != hipSuccess || occ < 1) occ = 1;
-    const int grid = min(nwork, ncu * occ);
-    hipLaunchKernelGGL(multi_kernel, dim3(grid), dim3(NT), 0, s, d_table, ndom, nwork);
+    // One group per work item, handed out by the hardware as CUs have room:
+    // items differ in cost (schemes, field counts, ragged chunks), and a
+    // resident grid of ncu * occupancy groups with a fixed share each ended
+    // with most CUs idle (48 subdomains of 48 to 192 columns a side, three
+    // SSP-RK3 stages: 13.18 -> 11.43 ms).
+    hipLaunchKernelGGL(multi_kernel, dim3(nwork), dim3(NT), 0, s, d_table, ndom);
     return hipGetLastError();
 }
 
