@@ -420,24 +420,28 @@ hipError_t launch_momentum_batch(const GridDev &g, int mom_ord, int lavisc, cons
     c.dy2 = (float)(1.0 / (2.0 * g.dy));
     c.dy3 = (float)(1.0 / (3.0 * g.dy));
     c.lavisc = lavisc;
-    // Levels per work item: the ring fill of an item (its first four levels)
-    // is paid once per chunk, so an item marches its whole column when the
-    // tiles alone fill the resident groups (four per CU); smaller grids split
-    // the columns into chunks of at least 32 levels.  At 512x512x160 whole
-    // columns are 4 % faster than 32-level chunks, and those 4 % faster than
-    // 16-level ones.
     const bool three_d = g.ny > 1;
     const int ntx3 = (g.nx - 5 + 31) / 32, nty3 = (g.ny - 5 + 7) / 8;
     const int tiles = three_d ? ntx3 * nty3 : (g.nx - 5 + 63) / 64;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
-        ncu = 256;
-    const int groups = 4 * ncu;
+    // Levels per work item: items run in rounds of four groups per CU (2D:
+    // sixteen), each taking as long as its levels and the ring fill, which
+    // measures like two more.  The length with the least rounds * (levels +
+    // fill) is taken, the longest of equals: a small grid marches one or two
+    // levels per item on all CUs, 1024 tiles march whole columns (4 % faster
+    // than 32-level items, which are 4 % faster than 16-level ones), and
+    // tiles that fill a round and a part of one are cut until the rounds are
+    // nearly full.  Tendencies of 20 fields, whole columns or at least 32
+    // levels -> this rule: 96x96x48 (36 tiles) 301 -> 196 us, 192x160x96 (120)
+    // 531 -> 468 us, 400x400x100 (650) 1142 -> 1049 us for 8 fields.
+    const long slots = (long)(three_d ? 4 : 16) * device_cus();
     int kchunk = g.nz;
-    if (tiles < groups) {
-        const int want = (groups + tiles - 1) / tiles;  // chunks per column
-        kchunk = std::min(g.nz, std::max(32, (g.nz + want - 1) / want));
+    long best = 0;
+    for (int k = g.nz; k >= 1; --k) {
+        const long rounds = ((long)tiles * ((g.nz + k - 1) / k) + slots - 1) / slots;
+        if (best == 0 || rounds * (k + 2) < best) {
+            best = rounds * (k + 2);
+            kchunk = k;
+        }
     }
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
     if (three_d) {
