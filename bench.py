@@ -582,7 +582,7 @@ def main():
     ap.add_argument("--tile-x", type=int, default=0, help="fused workload: columns of the tile (64, 16, or 32 with "
                                                        "--tile-y 8)")
     ap.add_argument("--blocks-per-cu", type=int, default=0,
-                    help="fused workload: at most this many workgroups per CU in a launch (0: one per work item)")
+                    help="fused workload: most workgroups per CU (0: as many as fit)")
     ap.add_argument("--no-graph", action="store_true")
     ap.add_argument("--no-variants", action="store_true", help="plain workload: skip the scheme variants")
     ap.add_argument("--copy-probe", type=int, default=0,

@@ -267,6 +267,7 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
     }
 }
 
+// items: work items per group of fpi fields; A.nwork counts all groups' items.
 // T: the precision of every field of the launch (FP64 and FP32 members of
 // a batch go to two launches, so that the FP32 kernel keeps the register
 // budget of FP32 arithmetic).
@@ -279,9 +280,17 @@ constexpr int fused_min_waves()
     return fused_six_waves<SCHEME, TX, TY, T>() ? 6 : 1;
 }
 
+// LDS of a work item: a field's tile and faces of one level, the chunk's velocities.
+template <int SCHEME, int TX, int TY, class T>
+constexpr int fused_lds_bytes()
+{
+    using I = Item<TX, TY, stencil_h<SCHEME>()>;
+    return (I::LH * I::LW + I::FS * I::NT) * (int)sizeof(T) + fused_kc<SCHEME, TX, TY, T>() * I::NV * (int)sizeof(float);
+}
+
 template <int SCHEME, int TX, int TY, class T>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(fused_min_waves<SCHEME, TX, TY, T>(), 8))) void
-fused_kernel(FusedArgs A)
+fused_kernel(FusedArgs A, int items, int fpi)
 {
     constexpr int H = stencil_h<SCHEME>();
     using I = Item<TX, TY, H>;
@@ -295,87 +304,86 @@ fused_kernel(FusedArgs A)
     const int tiles = A.ntx * A.nty;
     const int kc = A.kchunk;
 
-    for (int wi = blockIdx.x; wi < A.nwork; wi += gridDim.x) {
-        // XCD-aware order: consecutive work ids go round-robin over the 8
-        // XCDs; every XCD gets a contiguous range of tiles so that tile
-        // halos and velocity rows stay in one L2.
-        const int chunk = wi / tiles;
-        int t = wi - chunk * tiles;
-        if (A.xcd_remap) {
-            const int per = tiles / 8;
-            t = (t % 8) * per + t / 8;
+    // fields f0 .. f0 + fpi - 1 of the batch
+    const int fg = blockIdx.x / items, wi = blockIdx.x - fg * items;
+    const int f0 = fg * fpi;
+    // XCD-aware order: consecutive work ids go round-robin over the 8
+    // XCDs; every XCD gets a contiguous range of tiles so that tile
+    // halos and velocity rows stay in one L2.
+    const int chunk = wi / tiles;
+    int t = wi - chunk * tiles;
+    if (A.xcd_remap) {
+        const int per = tiles / 8;
+        t = (t % 8) * per + t / 8;
+    }
+    const int i0 = 4 + (t % A.ntx) * TX;
+    const int j0 = I::THREE_D ? 4 + (t / A.ntx) * TY : 1;
+    const int k0 = 1 + chunk * kc;
+    const int nk = min(kc, nz - k0 + 1);
+    const int i = i0 + tx, j = j0 + ty;
+    const bool valid = i <= nx - 2 && (!I::THREE_D || j <= ny - 2);
+    const int il = wrap(i, nx, A.mx), jl = I::THREE_D ? wrap(j, ny, A.my) : 1;
+    const int col = (il - 1) + nx * (jl - 1);
+    Slots<TX, TY, H> sl;
+    sl.init(tid, i0, j0, A);
+    // the chunk's face velocities and column w(k+1), read once for every
+    // field of the item: the source array and plane offset of each of this
+    // thread's staging slots are fixed, and all the chunk's loads are in
+    // flight together before they go to LDS
+    {
+        constexpr int VS = (I::NV + I::NT - 1) / I::NT;
+        const size_t plane = (size_t)nx * ny;
+        const float *vp[VS];
+        int voff[VS];
+        bool vw[VS];
+#pragma unroll
+        for (int s = 0; s < VS; ++s) {
+            const int e = tid + s * I::NT;
+            vp[s] = A.u;
+            voff[s] = -1;
+            vw[s] = false;
+            if (e < I::NF) {
+                int base, step;
+                size_t vcol;
+                const int kind = face_slot_geom<TX, TY, H>(e, i0, j0, A, base, step, vcol);
+                vp[s] = kind == 1 ? A.u : A.v;
+                voff[s] = (int)vcol;
+            } else if (e < I::NV) {
+                const int c = e - I::NF, cx = c % TX, cy = c / TX;
+                const int ci = wrap(i0 + cx, nx, A.mx), cj = I::THREE_D ? wrap(j0 + cy, ny, A.my) : 1;
+                vp[s] = A.w;  // w(k+1) at level k
+                voff[s] = (ci - 1) + nx * (cj - 1);
+                vw[s] = true;
+            }
         }
-        const int i0 = 4 + (t % A.ntx) * TX;
-        const int j0 = I::THREE_D ? 4 + (t / A.ntx) * TY : 1;
-        const int k0 = 1 + chunk * kc;
-        const int nk = min(kc, nz - k0 + 1);
-        const int i = i0 + tx, j = j0 + ty;
-        const bool valid = i <= nx - 2 && (!I::THREE_D || j <= ny - 2);
-        const int il = wrap(i, nx, A.mx), jl = I::THREE_D ? wrap(j, ny, A.my) : 1;
-        const int col = (il - 1) + nx * (jl - 1);
-        Slots<TX, TY, H> sl;
-        sl.init(tid, i0, j0, A);
-        // the chunk's face velocities and column w(k+1), read once for every
-        // field: the source array and plane offset of each of this thread's
-        // staging slots are fixed for the item, and all the chunk's loads are
-        // in flight together (issued before the barrier that waits for the
-        // previous item's fields) before they go to LDS
-        {
-            constexpr int VS = (I::NV + I::NT - 1) / I::NT;
-            const size_t plane = (size_t)nx * ny;
-            const float *vp[VS];
-            int voff[VS];
-            bool vw[VS];
+        float vb[KC][VS];
+#pragma unroll
+        for (int kk = 0; kk < KC; ++kk) {
+            const int k = k0 + kk;
 #pragma unroll
             for (int s = 0; s < VS; ++s) {
-                const int e = tid + s * I::NT;
-                vp[s] = A.u;
-                voff[s] = -1;
-                vw[s] = false;
-                if (e < I::NF) {
-                    int base, step;
-                    size_t vcol;
-                    const int kind = face_slot_geom<TX, TY, H>(e, i0, j0, A, base, step, vcol);
-                    vp[s] = kind == 1 ? A.u : A.v;
-                    voff[s] = (int)vcol;
-                } else if (e < I::NV) {
-                    const int c = e - I::NF, cx = c % TX, cy = c / TX;
-                    const int ci = wrap(i0 + cx, nx, A.mx), cj = I::THREE_D ? wrap(j0 + cy, ny, A.my) : 1;
-                    vp[s] = A.w;  // w(k+1) at level k
-                    voff[s] = (ci - 1) + nx * (cj - 1);
-                    vw[s] = true;
-                }
+                vb[kk][s] = 0.0f;
+                if (kk < nk && voff[s] >= 0 && (!vw[s] || k < nz))
+                    vb[kk][s] = vp[s][(size_t)(vw[s] ? k : k - 1) * plane + (size_t)voff[s]];
             }
-            float vb[KC][VS];
-#pragma unroll
-            for (int kk = 0; kk < KC; ++kk) {
-                const int k = k0 + kk;
-#pragma unroll
-                for (int s = 0; s < VS; ++s) {
-                    vb[kk][s] = 0.0f;
-                    if (kk < nk && voff[s] >= 0 && (!vw[s] || k < nz))
-                        vb[kk][s] = vp[s][(size_t)(vw[s] ? k : k - 1) * plane + (size_t)voff[s]];
-                }
-            }
-            __syncthreads();  // the previous item's fields are done with vel_lds
-#pragma unroll
-            for (int kk = 0; kk < KC; ++kk)
-#pragma unroll
-                for (int s = 0; s < VS; ++s)
-                    if (kk < nk && tid + s * I::NT < I::NV) vel_lds[kk * I::NV + tid + s * I::NT] = vb[kk][s];
-            __syncthreads();
         }
-        if constexpr (sizeof(T) == 8) {
+#pragma unroll
+        for (int kk = 0; kk < KC; ++kk)
+#pragma unroll
+            for (int s = 0; s < VS; ++s)
+                if (kk < nk && tid + s * I::NT < I::NV) vel_lds[kk * I::NV + tid + s * I::NT] = vb[kk][s];
+        __syncthreads();
+    }
+    if constexpr (sizeof(T) == 8) {
 #pragma unroll 1
-            for (int f = 0; f < A.n64_active; ++f)
-                march_field<SCHEME, TX, TY, T>(A, A.q64[f], A.q0_64[f], A.out64[f], tile_lds, face_lds, vel_lds, k0, nk,
-                                               i0, j0, tid, tx, ty, valid, col, sl);
-        } else {
+        for (int f = f0; f < min(A.n64_active, f0 + fpi); ++f)
+            march_field<SCHEME, TX, TY, T>(A, A.q64[f], A.q0_64[f], A.out64[f], tile_lds, face_lds, vel_lds, k0, nk,
+                                           i0, j0, tid, tx, ty, valid, col, sl);
+    } else {
 #pragma unroll 1
-            for (int f = 0; f < A.n32_active; ++f)
-                march_field<SCHEME, TX, TY, T>(A, A.q32[f], A.q0_32[f], A.out32[f], tile_lds, face_lds, vel_lds, k0, nk,
-                                               i0, j0, tid, tx, ty, valid, col, sl);
-        }
+        for (int f = f0; f < min(A.n32_active, f0 + fpi); ++f)
+            march_field<SCHEME, TX, TY, T>(A, A.q32[f], A.q0_32[f], A.out32[f], tile_lds, face_lds, vel_lds, k0, nk,
+                                           i0, j0, tid, tx, ty, valid, col, sl);
     }
 }
 
@@ -388,17 +396,46 @@ hipError_t launch_tiles(const FusedArgs &a0, hipStream_t s, int blocks_per_cu)
     const int tiles = A.ntx * A.nty;
     A.xcd_remap = (tiles % 8 == 0) ? 1 : 0;
     constexpr int KC = fused_kc<SCHEME, TX, TY, T>();
-    A.kchunk = A.kchunk <= 0 ? KC : min(A.kchunk, KC);
-    A.nwork = tiles * ((A.nz + A.kchunk - 1) / A.kchunk);
+    // A grid whose items leave the chip idle splits the batch: each item then
+    // marches fpi of the fields, so that FP32 launches have at least eight
+    // 256-thread groups per CU (what makes a few ragged rounds cheap) and
+    // FP64 ones the four that fit.  If one field per item does not give four
+    // groups per CU, the chunks are shortened to reach them (unless the caller
+    // set their length).  Every item stages the velocities of its chunk
+    // again, so larger grids keep all fields in one item (256x256x128:
+    // 1063 us, split further 1077).
+    // Tendencies of 20 fields, all fields per item -> this rule: 24x24x16
+    // 209 -> 86 us, 48x48x48 281 -> 171 us, 96x96x48 288 -> 207 us,
+    // 192x160x96 536 -> 483 us.
+    const int nf = sizeof(T) == 8 ? A.n64_active : A.n32_active;
+    const long cus = (long)device_cus() * 256 / (TX * TY);
+    const int kmax = A.kchunk <= 0 ? KC : min(A.kchunk, KC);
+    const auto chunks = [&](int kc) { return (A.nz + kc - 1) / kc; };
+    const long whole = (long)tiles * chunks(kmax), wide = (sizeof(T) == 8 ? 4 : 8) * cus;
+    const int split = (int)max(1L, min((long)nf, (wide + whole - 1) / whole));
+    const int fpi = (nf + split - 1) / split;
+    const int groups = (nf + fpi - 1) / fpi;
+    if (A.kchunk <= 0) {
+        const int nchunk = (int)max((long)chunks(kmax), min((long)A.nz, 4 * cus / ((long)tiles * groups)));
+        A.kchunk = (A.nz + nchunk - 1) / nchunk;
+    } else A.kchunk = kmax;
+    const int items = tiles * chunks(A.kchunk);
+    A.nwork = items * groups;
     // One group per work item: the hardware hands the next item to the CU
     // that has room first.  A resident grid of ncu * occupancy groups, each
     // taking every gridDim-th item, leaves most CUs idle behind the longest
     // share: a step of 20 fields at 512x512x160 (three stages, momenta
-    // included) took 18.55 ms that way and 16.02 ms this way.  Only a
-    // caller's limit of groups per CU asks for a smaller grid.
-    int grid = A.nwork;
-    if (blocks_per_cu > 0) grid = (int)min((long long)grid, (long long)device_cus() * blocks_per_cu);
-    hipLaunchKernelGGL((fused_kernel<SCHEME, TX, TY, T>), dim3(grid), dim3(TX * TY), 0, s, A);
+    // included) took 18.55 ms that way and 16.02 ms this way.  A caller's
+    // limit of groups per CU is kept by asking for that share of the LDS.
+    int dyn = 0;
+    if (blocks_per_cu > 0) {
+        int dev = 0, most = 0, lds = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+            hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) == hipSuccess)
+            dyn = max(0, min(most, lds / blocks_per_cu) - fused_lds_bytes<SCHEME, TX, TY, T>());
+    }
+    hipLaunchKernelGGL((fused_kernel<SCHEME, TX, TY, T>), dim3(A.nwork), dim3(TX * TY), dyn, s, A, items, fpi);
     return hipGetLastError();
 }
 

@@ -272,8 +272,8 @@ int mimadv_advection_1d(mimadv_ctx *ctx, const double *w0, const double *dens, i
 typedef struct mimadv_tuning {
     int group32;        /* FP32 fields per launch (default and maximum 18) */
     int kchunk;         /* levels per work item (default and maximum 8; 6 for FP32 WENO/MUSCL
-                           launches with 256-thread tiles) */
-    int blocks_per_cu;  /* persistent grid size per CU (default: occupancy) */
+                           launches with 256-thread tiles; small grids take fewer by default) */
+    int blocks_per_cu;  /* most workgroups per CU (default: as many as fit) */
     int tile_y;         /* rows of the column tile in 3D: 2, 4 or 8 */
     int tile_x;         /* columns of the tile: 64, 32 with tile_y 8 (or 0), or 16 with
                            tile_y 0 (16x16).  Both 0: 32x8 tiles in 3D; tile_x 0 with tile_y

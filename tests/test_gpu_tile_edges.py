@@ -150,3 +150,57 @@ def test_scalar_non_finite_values(cuda, scheme, lim, value):
         got = dx.cpu().numpy()
     assert not np.isfinite(got).all()
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+def _batch(cuda, mx, my, nz, nspec):
+    """Batch of momenta, two FP64 scalars and FP32 species on FP32-representable inputs."""
+    g, u, v, w, _ = case3d(mx, my, nz) if my else case2d(mx, nz)
+    u, v, w = (a.astype(np.float32) for a in (u, v, w))
+    rng = np.random.default_rng(17)
+    mom = [a * (1.0 + 0.1 * rng.standard_normal(a.shape)).astype(np.float32) for a in (u, v, w)]
+    f64 = [1.0 + rng.random(g.shape) for _ in range(2)]
+    f32 = [np.exp(rng.standard_normal(g.shape)).astype(np.float32) for _ in range(nspec)]
+    return g, _dev(cuda, u, v, w), _dev(cuda, *mom), _dev(cuda, *f64, *f32)
+
+
+@pytest.mark.parametrize("scheme", ["weno", "weno5", "muscl"])
+@pytest.mark.parametrize("dims", [(6, 6, 8), (33, 9, 17), (44, 37, 24), (130, 100, 40), (65, 0, 33)])
+def test_batch_field_split(cuda, scheme, dims):
+    """A batch whose fields are spread over work items, in whole or short chunks,
+    has the bits of each field advected alone and of chunks of a set length."""
+    print(f"case batch_field_split {scheme} {dims}", flush=True)
+    g, vel, _, fields = _batch(cuda, *dims, nspec=15)
+    with Advection(g, scal_adv=scheme, muscllimiter="MC") as a:
+        def run(which, kchunk):
+            a.set_tuning(kchunk=kchunk)
+            outs = [torch.zeros_like(f) for f in which]
+            a.batch_tendency(*vel, which, outs)
+            a.stream_sync()
+            return outs
+        base = run(fields, 0)
+        for kchunk in (5, 8):
+            for n, o in enumerate(run(fields, kchunk)):
+                assert torch.equal(o, base[n]), f"kchunk {kchunk} field {n}"
+        for n in (0, 1, 2, 9, 16):
+            assert torch.equal(run([fields[n]], 0)[0], base[n]), f"field {n} alone"
+
+
+@pytest.mark.parametrize("dims", [(33, 9, 17), (100, 90, 40), (139, 117, 33), (200, 190, 41)])
+def test_batch_momentum_chunk_lengths(cuda, dims):
+    """The FP32 momenta against the FP64 operator, whose bits are the oracle's,
+    where the dispatch takes one, two and more levels per work item.  Bound:
+    2e-6 of the field maximum, as for the other batched momenta."""
+    print(f"case batch_momentum_chunks {dims}", flush=True)
+    g, vel, mom, fields = _batch(cuda, *dims, nspec=1)
+    with Advection(g, scal_adv="weno") as a:
+        ref = [torch.zeros(g.shape, dtype=torch.float64, device=cuda) for _ in range(3)]
+        mom64, vel64 = [m.double() for m in mom], [x.double() for x in vel]  # alive until the sync
+        a.qnadv_uvw(0, mom64, vel64, ref)
+        ins = mom + fields
+        outs = [torch.zeros_like(f) for f in ins]
+        a.batch_tendency(*vel, ins, outs, momentum=True)
+        a.stream_sync()
+        I = g.interior()
+        for c in range(3):
+            want, got = -ref[c][I], outs[c].double()[I]
+            assert float((got - want).abs().max() / want.abs().max()) <= 2e-6, f"component {c}"
