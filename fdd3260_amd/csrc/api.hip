@@ -533,19 +533,20 @@ int mimadv_fill_halo(mimadv_ctx *c, int nf, double *const *x, unsigned flags)
 {
     if (!c) return MIMADV_ERR_ARG;
     if (nf < 0 || (nf > 0 && !x)) return fail(c, MIMADV_ERR_ARG, "bad field list");
+    for (int f = 0; f < nf; ++f)
+        if (!x[f]) return fail(c, MIMADV_ERR_ARG, "field pointer is NULL");
+    if (!(flags & MIMADV_HOST_PTRS)) {
+        HIPCHK(c, launch_fill_scalars(c->g, nf, x, c->stream));
+        return MIMADV_OK;
+    }
     size_t bytes = c->n3() * sizeof(double);
     for (int f = 0; f < nf; ++f) {
-        if (!x[f]) return fail(c, MIMADV_ERR_ARG, "field pointer is NULL");
-        if (flags & MIMADV_HOST_PTRS) {
-            int rc = ensure_stage(c, 1);
-            if (rc) return rc;
-            HIPCHK(c, hipMemcpyAsync(c->stage, x[f], bytes, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(c, launch_fill_scalar(c->g, c->stage, c->stream));
-            HIPCHK(c, hipMemcpyAsync(x[f], c->stage, bytes, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-        } else {
-            HIPCHK(c, launch_fill_scalar(c->g, x[f], c->stream));
-        }
+        int rc = ensure_stage(c, 1);
+        if (rc) return rc;
+        HIPCHK(c, hipMemcpyAsync(c->stage, x[f], bytes, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, launch_fill_scalars(c->g, 1, &c->stage, c->stream));
+        HIPCHK(c, hipMemcpyAsync(x[f], c->stage, bytes, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
     }
     return MIMADV_OK;
 }
@@ -1516,6 +1517,7 @@ int mimadv_advection_1d(mimadv_ctx *c, const double *w0, const double *dens, int
         int rc = ensure_stage(c, 3);
         if (rc) return rc;
         double *sq = c->stage, *sx = c->stage + c->n3(), *sd = c->stage + 2 * c->n3();
+        const double *sqc = sq;
         if (d3) {
             HIPCHK(c, hipMemcpyAsync(sd, d3, bytes, hipMemcpyHostToDevice, c->stream));
             d3 = sd;
@@ -1523,13 +1525,13 @@ int mimadv_advection_1d(mimadv_ctx *c, const double *w0, const double *dens, int
         for (int f = 0; f < nf; ++f) {
             HIPCHK(c, hipMemcpyAsync(sq, q[f], bytes, hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipMemcpyAsync(sx, xs[f], bytes, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(c, launch_advection_1d(c->g, c->d_w0, dprof, d3, sq, sx, c->stream));
+            HIPCHK(c, launch_advection_1d(c->g, c->d_w0, dprof, d3, 1, &sqc, &sx, c->stream));
             HIPCHK(c, hipMemcpyAsync(xs[f], sx, bytes, hipMemcpyDeviceToHost, c->stream));
         }
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return MIMADV_OK;
     }
-    for (int f = 0; f < nf; ++f) HIPCHK(c, launch_advection_1d(c->g, c->d_w0, dprof, d3, q[f], xs[f], c->stream));
+    HIPCHK(c, launch_advection_1d(c->g, c->d_w0, dprof, d3, nf, q, xs, c->stream));
     return MIMADV_OK;
 }
 

@@ -123,7 +123,8 @@ struct MomBatchArgs {
     int epi, fill;
 };
 hipError_t launch_momentum_batch(const GridDev &g, int mom_ord, int lavisc, const MomBatchArgs &a, hipStream_t s);
-hipError_t launch_fill_scalar(const GridDev &g, double *x, hipStream_t s);
+// qnbc_p4 of nf scalars
+hipError_t launch_fill_scalars(const GridDev &g, int nf, double *const *x, hipStream_t s);
 // lbcu_p4 of a single-tile run (u, v, w; v unused in 2D)
 hipError_t launch_fill_winds(const GridDev &g, double *u, double *v, double *w, hipStream_t s);
 // integ_mom of one component (tw = the sponge factor for w, 1 otherwise)
@@ -134,10 +135,10 @@ hipError_t launch_integ_mom(const GridDev &g, int sorder, int im, double dt, dou
                             const double *const *a, double *const *tend, double *const *x, hipStream_t s);
 // the reference's implicit sponge factor of integ_mom (host, FP64)
 double sponge_factor(int nz, int sorder, int im, double dt, const double *z0, double zmax, double zdamp, int sponge);
-// xs -= dref*w0*grad_1d(q/dref) on interior columns; dref = d3 (3D) if not
+// xs -= dref*w0*grad_1d(q/dref) of nf fields on interior columns; dref = d3 (3D) if not
 // NULL, else dprof (levels) if not NULL, else 1 (util.hip)
-hipError_t launch_advection_1d(const GridDev &g, const double *w0, const double *dprof, const double *d3,
-                               const double *q, double *xs, hipStream_t s);
+hipError_t launch_advection_1d(const GridDev &g, const double *w0, const double *dprof, const double *d3, int nf,
+                               const double *const *q, double *const *xs, hipStream_t s);
 hipError_t launch_integ_scal(long n, int sorder, int im, double dt, const double *xold, const double *a,
                              double *tend, double *x, hipStream_t s);
 hipError_t launch_totalav(const GridDev &g, const double *x, double *d_out2, hipStream_t s);
@@ -146,7 +147,6 @@ hipError_t launch_level_scale(const GridDev &g, const double *prof, const double
                               double shift, hipStream_t s);
 // q = q*d or q/d elementwise
 hipError_t launch_field_scale(const GridDev &g, double *q, const double *d, int divide, hipStream_t s);
-hipError_t launch_wsum(const GridDev &g, const void *x, bool fp32, double *d_part, double *d_out, hipStream_t s);
 
 // Domain budgets (dzw-weighted interior sums) of up to BUDGET_MAXF fields in
 // two launches: per-block partials reduced with wavefront shuffles, then one

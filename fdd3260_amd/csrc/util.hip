@@ -1,6 +1,7 @@
 // util.hip -- ghost fill, stage combine and interior reductions.
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <mutex>
 
 #include "mimadv_internal.hpp"
@@ -9,38 +10,40 @@ namespace mimadv {
 
 namespace {
 
-// qnbc_p4 (bc.f90:378-503), serial branch.  The reference runs the x copy,
-// then the y copy over full rows, then the z copy, then the mirror fills;
-// each pass is one launch here so later passes see earlier results.
-__global__ void fill_x_kernel(int nx, int ny, int nz, int bc_w, int bc_e, double *x)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int k = blockIdx.y + 1;
-    if (j > ny) return;
-    double *r = x + (size_t)nx * ((size_t)(j - 1) + (size_t)ny * (k - 1));
-    auto X = [&](int i) -> double & { return r[i - 1]; };
-    if (bc_w == 0 || bc_e == 0) {
-        X(1) = X(nx - 4);
-        X(2) = X(nx - 3);
-        X(3) = X(nx - 2);
-        X(nx) = X(5);
-        X(nx - 1) = X(4);
-    }
-}
+// Fields of one launch at most.
+constexpr int FIELDS_MAX = 8;
+struct FieldList {
+    double *p[FIELDS_MAX];
+};
 
-__global__ void fill_y_kernel(int nx, int ny, int nz, double *x)
+// qnbc_p4 (bc.f90:378-503), serial branch.  The reference runs the x copy,
+// then the y copy over full rows, then the z copy, then the mirror fills.
+// Sides have at least eleven points (mimadv_create), so the sources of the
+// periodic x and y copies are interior points, and one launch writes every
+// ghost column of a plane from its wrapped one, for several fields at once.
+// Launches bound these fills (3 us each at 64x64x48): three winds and twelve
+// scalars took 30 of them, now 3 of 3 us each.
+__global__ __launch_bounds__(256) void fill_xy_kernel(int nx, int ny, int per_x, int per_y, FieldList l)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int k = blockIdx.y + 1;
-    if (i > nx) return;
-    size_t sy = (size_t)nx;
-    double *c = x + (size_t)(i - 1) + (size_t)nx * ny * (k - 1);
-    auto X = [&](int j) -> double & { return c[sy * (j - 1)]; };
-    X(1) = X(ny - 4);
-    X(2) = X(ny - 3);
-    X(3) = X(ny - 2);
-    X(ny) = X(5);
-    X(ny - 1) = X(4);
+    double *x = l.p[blockIdx.z] + (size_t)nx * ny * blockIdx.y;
+    const int rows = per_y ? ny - 5 : ny;  // rows that only the x copy writes
+    const int e = blockIdx.x * 256 + threadIdx.x, ex = per_x ? 5 * rows : 0;
+    int i, j;
+    if (e < ex) {
+        const int r = e / 5, g = e - 5 * r;
+        i = g < 3 ? g + 1 : nx - 4 + g;
+        j = per_y ? r + 4 : r + 1;
+    } else {
+        const int g = (e - ex) / nx;
+        if (!per_y || g >= 5) return;
+        i = e - ex - g * nx + 1;
+        j = g < 3 ? g + 1 : ny - 4 + g;
+    }
+    const auto from = [](int p, int n, int per) {
+        if (!per) return p;
+        return p <= 3 ? p + n - 5 : (p >= n - 1 ? p - (n - 5) : p);
+    };
+    x[(i - 1) + (size_t)nx * (j - 1)] = x[(from(i, nx, per_x) - 1) + (size_t)nx * (from(j, ny, per_y) - 1)];
 }
 
 __global__ void fill_z_kernel(int nx, int ny, int nz, double *x)
@@ -148,21 +151,38 @@ __global__ void integ_kernel(long n, int sorder, double a_lm, double b_lm, doubl
     }
 }
 
-// Interior sums per level: plain and dzw-weighted, tree reduction within a
-// block (deterministic), one block per level.
+// Interior sums per level, one block per level: every thread adds its cells in
+// the order t, t + 256, ... of the level's interior, eight loads in flight
+// and no division per cell (8.5 -> 4.1 us at 64x64x48), and a tree of fixed
+// shape joins the 256 sums (deterministic).
 __global__ __launch_bounds__(256) void level_sums_kernel(int nx, int ny, int nz, const double *__restrict__ x,
                                                          double *__restrict__ part)
 {
     const bool three_d = ny > 1;
-    int k = blockIdx.x + 1;
-    int j0 = three_d ? 4 : 1, j1 = three_d ? ny - 2 : 1;
-    int mx = nx - 5, my = j1 - j0 + 1;
-    long cnt = (long)mx * my;
-    const double *p = x + (size_t)nx * ny * (k - 1);
+    const int k = blockIdx.x + 1;
+    const int j0 = three_d ? 4 : 1, j1 = three_d ? ny - 2 : 1;
+    const int mx = nx - 5, my = j1 - j0 + 1;
+    const long cnt = (long)mx * my;
+    const double *p = x + (size_t)nx * ny * (k - 1) + 3 + (size_t)nx * (j0 - 1);
+    // 256 cells on: so many rows and columns
+    const int dj = 256 / mx, di = 256 - dj * mx;
+    int jj = threadIdx.x / mx, ii = threadIdx.x - jj * mx;
     double s = 0.0;
-    for (long t = threadIdx.x; t < cnt; t += blockDim.x) {
-        int jj = (int)(t / mx), ii = (int)(t - (long)jj * mx);
-        s += p[(size_t)(ii + 3) + (size_t)nx * (jj + j0 - 1)];
+    for (long t = threadIdx.x; t < cnt; t += 8 * 256) {
+        double v[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            v[m] = t + m * 256 < cnt ? p[ii + (size_t)nx * jj] : 0.0;
+            ii += di;
+            jj += dj;
+            if (ii >= mx) {
+                ii -= mx;
+                ++jj;
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            if (t + m * 256 < cnt) s += v[m];
     }
     __shared__ double sh[256];
     sh[threadIdx.x] = s;
@@ -174,57 +194,30 @@ __global__ __launch_bounds__(256) void level_sums_kernel(int nx, int ny, int nz,
     if (threadIdx.x == 0) part[k - 1] = sh[0];
 }
 
-__global__ void finish_sums_kernel(int nz, long ncells, const double *__restrict__ part, const double *__restrict__ dzw,
-                                   double *__restrict__ out)
+// One wave: the level sums are read side by side and added in level order
+// (5.1 -> 2.6 us for 48 levels).
+__global__ __launch_bounds__(64) void finish_sums_kernel(int nz, long ncells, const double *__restrict__ part,
+                                                         const double *__restrict__ dzw, double *__restrict__ out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    __shared__ double sp[64], sz[64];
     double s = 0.0, sw = 0.0;
-    for (int k = 0; k < nz; ++k) {
-        s += part[k];
-        sw += dzw[k] * part[k];
-    }
-    out[0] = s / (double)ncells;
-    out[1] = sw;
-}
-
-// dzw-weighted interior sum per level of an FP32 or FP64 field (FP64
-// accumulation, deterministic tree)
-template <class T>
-__global__ __launch_bounds__(256) void level_wsums_kernel(int nx, int ny, int nz, const T *__restrict__ x,
-                                                          const double *__restrict__ dzw, double *__restrict__ part)
-{
-    const bool three_d = ny > 1;
-    int k = blockIdx.x + 1;
-    int j0 = three_d ? 4 : 1, j1 = three_d ? ny - 2 : 1;
-    int mx = nx - 5, my = j1 - j0 + 1;
-    long cnt = (long)mx * my;
-    const T *p = x + (size_t)nx * ny * (k - 1);
-    double s = 0.0;
-    for (long t = threadIdx.x; t < cnt; t += blockDim.x) {
-        int jj = (int)(t / mx), ii = (int)(t - (long)jj * mx);
-        s += double(p[(size_t)(ii + 3) + (size_t)nx * (jj + j0 - 1)]);
-    }
-    __shared__ double sh[256];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+    for (int k0 = 0; k0 < nz; k0 += 64) {
+        const int k = k0 + threadIdx.x;
+        sp[threadIdx.x] = k < nz ? part[k] : 0.0;
+        sz[threadIdx.x] = k < nz ? dzw[k] : 0.0;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int n = 0; n < min(64, nz - k0); ++n) {
+                s += sp[n];
+                sw += sz[n] * sp[n];
+            }
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[k - 1] = dzw[k - 1] * sh[0];
+    if (threadIdx.x == 0) {
+        out[0] = s / (double)ncells;
+        out[1] = sw;
+    }
 }
-
-__global__ void sum_levels_kernel(int nz, const double *__restrict__ part, double *__restrict__ out)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0;
-    for (int k = 0; k < nz; ++k) s += part[k];
-    out[0] = s;
-}
-
-}  // namespace
-
-namespace {
 
 // Sum over the 64 lanes of a wavefront with cross-lane shuffles (no LDS,
 // no barrier); the order of the butterfly is fixed, so the result is
@@ -322,34 +315,54 @@ hipError_t launch_budgets(const BudgetArgs &a, int nf, double *d_out, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_wsum(const GridDev &g, const void *x, bool fp32, double *d_part, double *d_out, hipStream_t s)
+namespace {
+
+// Whether two arrays of n values share none of them.
+bool apart(const double *a, const double *b, size_t n)
 {
-    if (fp32)
-        hipLaunchKernelGGL(level_wsums_kernel<float>, dim3(g.nz), dim3(256), 0, s, g.nx, g.ny, g.nz, (const float *)x,
-                           g.zm.dzw, d_part);
-    else
-        hipLaunchKernelGGL(level_wsums_kernel<double>, dim3(g.nz), dim3(256), 0, s, g.nx, g.ny, g.nz,
-                           (const double *)x, g.zm.dzw, d_part);
-    hipLaunchKernelGGL(sum_levels_kernel, dim3(1), dim3(64), 0, s, g.nz, d_part, d_out);
-    return hipGetLastError();
+    const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+    return (p < q ? q - p : p - q) >= n * sizeof(double);
 }
 
-hipError_t launch_fill_scalar(const GridDev &g, double *x, hipStream_t s)
+// The periodic x and y copies of nf fields.
+void fill_xy(const GridDev &g, int nf, double *const *x, hipStream_t s)
+{
+    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int per_x = g.bcl[0] == 0 || g.bcl[1] == 0, per_y = ny > 1 && (g.bcl[2] == 0 || g.bcl[3] == 0);
+    if (!per_x && !per_y) return;
+    const int n = (per_x ? 5 * (per_y ? ny - 5 : ny) : 0) + (per_y ? 5 * nx : 0);
+    for (int f0 = 0; f0 < nf;) {
+        int n1 = std::min(FIELDS_MAX, nf - f0);
+        for (int f = 1; f < n1; ++f)
+            for (int h = 0; h < f; ++h)
+                if (!apart(x[f0 + f], x[f0 + h], (size_t)nx * ny * nz)) n1 = f;
+        FieldList l = {};
+        for (int f = 0; f < n1; ++f) l.p[f] = x[f0 + f];
+        hipLaunchKernelGGL(fill_xy_kernel, dim3((n + 255) / 256, nz, n1), dim3(256), 0, s, nx, ny, per_x, per_y, l);
+        f0 += n1;
+    }
+}
+
+}  // namespace
+
+hipError_t launch_fill_scalars(const GridDev &g, int nf, double *const *xs, hipStream_t s)
 {
     int nx = g.nx, ny = g.ny, nz = g.nz;
     bool three_d = ny > 1;
-    if (g.bcl[0] == 0 || g.bcl[1] == 0)
-        hipLaunchKernelGGL(fill_x_kernel, dim3((ny + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, g.bcl[0], g.bcl[1], x);
-    if (three_d && (g.bcl[2] == 0 || g.bcl[3] == 0))
-        hipLaunchKernelGGL(fill_y_kernel, dim3((nx + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, x);
-    if (g.bcl[4] == 0 || g.bcl[5] == 0) {
-        size_t n = (size_t)nx * ny;
-        hipLaunchKernelGGL(fill_z_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, nx, ny, nz, x);
+    fill_xy(g, nf, xs, s);
+    for (int f = 0; f < nf; ++f) {
+        double *x = xs[f];
+        if (g.bcl[4] == 0 || g.bcl[5] == 0) {
+            size_t n = (size_t)nx * ny;
+            hipLaunchKernelGGL(fill_z_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, nx, ny, nz, x);
+        }
+        if (g.bcl[0] != 0 || g.bcl[1] != 0)
+            hipLaunchKernelGGL(mirror_x_kernel, dim3((ny + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, g.bcl[0],
+                               g.bcl[1], x);
+        if (three_d && (g.bcl[2] != 0 || g.bcl[3] != 0))
+            hipLaunchKernelGGL(mirror_y_kernel, dim3((nx + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, g.bcl[2],
+                               g.bcl[3], x);
     }
-    if (g.bcl[0] != 0 || g.bcl[1] != 0)
-        hipLaunchKernelGGL(mirror_x_kernel, dim3((ny + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, g.bcl[0], g.bcl[1], x);
-    if (three_d && (g.bcl[2] != 0 || g.bcl[3] != 0))
-        hipLaunchKernelGGL(mirror_y_kernel, dim3((nx + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, g.bcl[2], g.bcl[3], x);
     return hipGetLastError();
 }
 
@@ -357,19 +370,15 @@ hipError_t launch_fill_winds(const GridDev &g, double *u, double *v, double *w, 
 {
     int nx = g.nx, ny = g.ny, nz = g.nz;
     bool three_d = ny > 1;
-    double *f[3] = {u, three_d ? v : nullptr, w};
+    double *f[3] = {u, three_d ? v : w, w};
+    const int nf = three_d ? 3 : 2;
     // periodic copies in x, y, z (each pass sees the previous ones), then
     // the normal-component fills of the non-periodic sides
-    for (double *x : f)
-        if (x && (g.bcl[0] == 0 || g.bcl[1] == 0))
-            hipLaunchKernelGGL(fill_x_kernel, dim3((ny + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, 0, 0, x);
-    for (double *x : f)
-        if (x && three_d && (g.bcl[2] == 0 || g.bcl[3] == 0))
-            hipLaunchKernelGGL(fill_y_kernel, dim3((nx + 63) / 64, nz), dim3(64), 0, s, nx, ny, nz, x);
-    for (double *x : f)
-        if (x && (g.bcl[4] == 0 || g.bcl[5] == 0)) {
+    fill_xy(g, nf, f, s);
+    if (g.bcl[4] == 0 || g.bcl[5] == 0)
+        for (int c = 0; c < nf; ++c) {
             size_t n = (size_t)nx * ny;
-            hipLaunchKernelGGL(fill_z_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, nx, ny, nz, x);
+            hipLaunchKernelGGL(fill_z_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, nx, ny, nz, f[c]);
         }
     if (g.bcl[0] != 0 || g.bcl[1] != 0) {
         // u along x: one line per (j, k)
@@ -507,23 +516,37 @@ namespace {
 // 400-473): xs(i,j,k) -= dref(k)*w0(k)*gz(k), gz(k) the derivative at level
 // k of the quadratic through the values x/dref of levels k-1, k, k+1 (the
 // floor reads x(1) at distance dz*fdz0(1); gz(nz) = 0).  One thread per
-// interior column, marching up with a three-level register window.
-__global__ __launch_bounds__(64) void adv1d_kernel(GridDev g, const double *__restrict__ w0,
+// interior column, field and chunk of levels, marching up with a three-level
+// register window.  Memory latency bounds it: a column is a serial chain of
+// loads and divisions, so small grids take short chunks (each repeats two
+// divisions) and all fields go in one launch: six fields at 64x64x48, whole
+// columns and a launch each 6 * 34 us -> 10.6 us.
+struct Adv1dArgs {
+    const double *q[FIELDS_MAX];
+    double *xs[FIELDS_MAX];
+};
+
+__global__ __launch_bounds__(64) void adv1d_kernel(GridDev g, const double *__restrict__ w0_,
                                                    const double *__restrict__ dprof, const double *__restrict__ d3,
-                                                   const double *__restrict__ q, double *__restrict__ xs)
+                                                   Adv1dArgs a, int nf, int kchunk)
 {
     const int nx = g.nx, ny = g.ny, nz = g.nz;
     const bool three_d = ny > 1;
-    const int i = 4 + blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = 4 + blockIdx.x * 64 + threadIdx.x;
     const int j = three_d ? 4 + (int)blockIdx.y : 1;
     if (i > nx - 2) return;
+    const int chunk = blockIdx.z / nf, f = blockIdx.z - chunk * nf;
+    const double *__restrict__ q = a.q[f];
+    double *__restrict__ xs = a.xs[f];
+    const int k0 = 1 + chunk * kchunk, k1 = min(nz, k0 + kchunk - 1);
     const size_t plane = (size_t)nx * ny, col = (size_t)(i - 1) + (size_t)nx * (j - 1);
-    const double *fdz0 = g.zm.fdz0;
+    const auto fdz0 = table(g.zm.fdz0), w0 = table(w0_), dp = table(dprof);
     const double dz = g.zm.dz;
-    auto dref = [&](int k) { return d3 ? d3[col + (size_t)(k - 1) * plane] : (dprof ? dprof[k - 1] : 1.0); };
-    double dk = dref(1);
-    double x0 = q[col] / dk, xm = 0.0;
-    for (int k = 1; k <= nz; ++k) {
+    auto dref = [&](int k) { return d3 ? d3[col + (size_t)(k - 1) * plane] : (dprof ? dp[k - 1] : 1.0); };
+    double dk = dref(k0);
+    double x0 = q[col + (size_t)(k0 - 1) * plane] / dk;
+    double xm = k0 > 1 ? q[col + (size_t)(k0 - 2) * plane] / dref(k0 - 1) : 0.0;
+    for (int k = k0; k <= k1; ++k) {
         double gz = 0.0, dn = 0.0, xp = 0.0;
         if (k <= nz - 1) {
             dn = dref(k + 1);
@@ -547,11 +570,36 @@ __global__ __launch_bounds__(64) void adv1d_kernel(GridDev g, const double *__re
 
 }  // namespace
 
-hipError_t launch_advection_1d(const GridDev &g, const double *w0, const double *dprof, const double *d3,
-                               const double *q, double *xs, hipStream_t s)
+hipError_t launch_advection_1d(const GridDev &g, const double *w0, const double *dprof, const double *d3, int nf,
+                               const double *const *q, double *const *xs, hipStream_t s)
 {
-    const int mx = g.nx - 5, my = g.ny > 1 ? g.ny - 5 : 1;
-    hipLaunchKernelGGL(adv1d_kernel, dim3((mx + 63) / 64, my, 1), dim3(64), 0, s, g, w0, dprof, d3, q, xs);
+    const int mx = g.nx - 5, my = g.ny > 1 ? g.ny - 5 : 1, ntx = (mx + 63) / 64;
+    // Fields go together while no tendency overlaps another field's arrays (a
+    // list may add to one tendency twice); a tendency over its own inputs is
+    // marched in one chunk, which reads each level before it writes it.
+    const size_t n3 = (size_t)g.nx * g.ny * g.nz;
+    const auto free_of = [&](int f, int h) {  // the tendency of f and the inputs of h
+        return apart(xs[f], q[h], n3) && (!d3 || apart(xs[f], d3, n3));
+    };
+    for (int f0 = 0; f0 < nf;) {
+        const bool chunked = free_of(f0, f0);
+        int n1 = 1;
+        for (bool ok = chunked; ok && n1 < FIELDS_MAX && f0 + n1 < nf; n1 += ok) {
+            const int f = f0 + n1;
+            ok = free_of(f, f);
+            for (int h = f0; h < f; ++h)
+                ok = ok && apart(xs[f], xs[h], n3) && free_of(f, h) && free_of(h, f);
+        }
+        Adv1dArgs a = {};
+        for (int f = 0; f < n1; ++f) {
+            a.q[f] = q[f0 + f];
+            a.xs[f] = xs[f0 + f];
+        }
+        const int kchunk = chunked ? levels_per_item(g.nz, (long)ntx * my * n1, 16, 16) : g.nz;
+        hipLaunchKernelGGL(adv1d_kernel, dim3(ntx, my, n1 * ((g.nz + kchunk - 1) / kchunk)), dim3(64), 0, s, g, w0,
+                           dprof, d3, a, n1, kchunk);
+        f0 += n1;
+    }
     return hipGetLastError();
 }
 

@@ -204,3 +204,69 @@ def test_batch_momentum_chunk_lengths(cuda, dims):
         for c in range(3):
             want, got = -ref[c][I], outs[c].double()[I]
             assert float((got - want).abs().max() / want.abs().max()) <= 2e-6, f"component {c}"
+
+
+@pytest.mark.parametrize("dims", [(6, 6, 8), (7, 45, 9), (251, 9, 8), (60, 0, 9)])
+@pytest.mark.parametrize("sides", [("per", "per", "per", "per"), ("per", "per", "nnf", "ope"),
+                                   ("ope", "nnf", "per", "per")])
+def test_fill_of_many_fields(cuda, dims, sides):
+    """Ghosts of a list of fields, more than one launch takes and one of them
+    listed twice, next to the oracle's of each field."""
+    print(f"case fill_many {dims} {sides}", flush=True)
+    mx, my, nz = dims
+    bcl = sides + ("nnf", "nnf")
+    g = (case3d(mx, my, nz, bcl=bcl) if my else case2d(mx, nz, bcl=bcl))[0]
+    rng = np.random.default_rng(3)
+    xs = [rng.standard_normal(g.shape) for _ in range(11)]
+    with Advection(g) as a:
+        d = _dev(cuda, *xs)
+        a.fill_halo(d[:4] + [d[2]] + d[4:])
+        a.stream_sync()
+    ora = Oracle(g)
+    for n, x in enumerate(xs):
+        ora.fill_scalar(x)
+        assert np.array_equal(d[n].cpu().numpy(), x), f"field {n}"
+
+
+@pytest.mark.parametrize("dims", [(6, 6, 8), (64, 9, 33), (130, 65, 40), (60, 0, 33)])
+def test_advection_1d_of_many_fields(cuda, dims):
+    """Lists longer than a launch takes, one tendency listed twice (both
+    fields add to it in order) and one field that is its own tendency."""
+    print(f"case advection_1d_many {dims}", flush=True)
+    mx, my, nz = dims
+    g = (case3d(mx, my, nz) if my else case2d(mx, nz))[0]
+    rng = np.random.default_rng(8)
+    w0 = rng.standard_normal(g.nz)
+    qs = [rng.standard_normal(g.shape) for _ in range(11)]
+    ts = [rng.standard_normal(g.shape) for _ in range(11)]
+    dens = 1.0 + rng.random(g.shape)
+    qi, ti = list(range(11)) + [3], list(range(11)) + [4]
+    with Advection(g) as a:
+        dq, dt, dd = _dev(cuda, *qs), _dev(cuda, *ts), _dev(cuda, dens)[0]
+        a.advection_1d(w0, [dq[n] for n in qi] + [dq[0]], [dt[n] for n in ti] + [dq[0]], dens=dd)
+        a.stream_sync()
+    ora = Oracle(g)
+    for n, m in zip(qi, ti):
+        ora.advection_1d(w0, qs[n], ts[m], dref3=dens)
+    own = qs[0].copy()
+    ora.advection_1d(w0, qs[0], own, dref3=dens)
+    for n in range(11):
+        assert np.array_equal(dt[n].cpu().numpy(), ts[n]), f"tendency {n}"
+    assert np.array_equal(dq[0].cpu().numpy(), own)
+
+
+@pytest.mark.parametrize("dims", [(6, 6, 8), (17, 15, 65), (256, 9, 8), (300, 130, 9), (6, 0, 8), (600, 0, 130)])
+def test_totalav_sizes(cuda, dims):
+    """Mean and budget next to sums in extended precision; n additions of
+    positive values are within n units of round-off, relatively."""
+    print(f"case totalav {dims}", flush=True)
+    mx, my, nz = dims
+    g = (case3d(mx, my, nz) if my else case2d(mx, nz))[0]
+    x = np.random.default_rng(5).random(g.shape)
+    with Advection(g) as a:
+        mean, budget = a.totalav(_dev(cuda, x)[0])
+    inner = x[g.interior()].astype(np.longdouble)
+    tol = inner.size * 2.0 ** -53
+    assert abs(mean - float(inner.mean())) <= tol * mean
+    want = float((inner.reshape(nz, -1).sum(axis=1) * np.asarray(g.dzw, dtype=np.longdouble)).sum())
+    assert abs(budget - want) <= tol * want
