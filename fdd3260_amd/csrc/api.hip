@@ -218,6 +218,7 @@ int advance_steps(mimadv_ctx *c, int integrator, int nsteps, double dt, const do
     // The scratch arrays need no start values: a stage writes its whole output,
     // every ghost being the periodic image of an interior value, and the
     // accumulated tendency is written before it is read, on interior cells only.
+    ScalarArgs args[SCALAR_FIELDS];
     for (int s = 0; s < nsteps; ++s) {
         if (integrator == MIMADV_INT_EULER) {
             // sorder = 1 (integ.h): x = xold + dt*a, into w1, then back
@@ -237,7 +238,7 @@ int advance_steps(mimadv_ctx *c, int integrator, int nsteps, double dt, const do
                 a.qn = w1;
                 a.b_lm = 0.0;
                 a.adt = dt;
-                HIPCHK(c, launch_scalar_fp64(c->g, sp, a, c->stream));
+                HIPCHK(c, launch_scalar_fp64(c->g, sp, &a, 1, c->stream));
                 HIPCHK(c, hipMemcpyAsync(q[f], w1, n3 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
             }
             continue;
@@ -245,8 +246,9 @@ int advance_steps(mimadv_ctx *c, int integrator, int nsteps, double dt, const do
         int nst = integrator == MIMADV_INT_HEUN ? 2 : 3;
         for (int st = 1; st <= nst; ++st) {
             for (int f = 0; f < nf; ++f) {
+                ScalarArgs &a = args[f % SCALAR_FIELDS];
                 double *w1 = c->work + (2 * f) * n3, *w2 = c->work + (2 * f + 1) * n3;
-                ScalarArgs a{};
+                a = ScalarArgs{};
                 a.u = u;
                 a.v = v;
                 a.w = w;
@@ -281,7 +283,8 @@ int advance_steps(mimadv_ctx *c, int integrator, int nsteps, double dt, const do
                         a.q = w2; a.qn = q[f]; a.c0 = 1.0 / 3.0; a.c1 = 2.0 / 3.0;
                     }
                 }
-                HIPCHK(c, launch_scalar_fp64(c->g, sp, a, c->stream));
+                const int n = f % SCALAR_FIELDS + 1;
+                if (n == SCALAR_FIELDS || f == nf - 1) HIPCHK(c, launch_scalar_fp64(c->g, sp, args, n, c->stream));
             }
         }
     }
@@ -450,8 +453,10 @@ int mimadv_scalar_tendency(mimadv_ctx *c, double dt0, const double *u, const dou
     }
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     float kms_total = 0.0f;
+    ScalarArgs args[SCALAR_FIELDS];
     for (int f = 0; f < nf; ++f) {
-        ScalarArgs a{};
+        ScalarArgs &a = args[f % SCALAR_FIELDS];
+        a = ScalarArgs{};
         a.u = du;
         a.v = dv;
         a.w = dw;
@@ -468,7 +473,7 @@ int mimadv_scalar_tendency(mimadv_ctx *c, double dt0, const double *u, const dou
             a.q = sq;
             a.xs = sx;
             HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-            HIPCHK(c, launch_scalar_fp64(c->g, sp, a, c->stream));
+            HIPCHK(c, launch_scalar_fp64(c->g, sp, &a, 1, c->stream));
             HIPCHK(c, hipEventRecord(c->ev1, c->stream));
             HIPCHK(c, hipMemcpyAsync(xs[f], sx, bytes, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -478,7 +483,8 @@ int mimadv_scalar_tendency(mimadv_ctx *c, double dt0, const double *u, const dou
         } else {
             a.q = q[f];
             a.xs = xs[f];
-            HIPCHK(c, launch_scalar_fp64(c->g, sp, a, c->stream));
+            const int n = f % SCALAR_FIELDS + 1;
+            if (n == SCALAR_FIELDS || f == nf - 1) HIPCHK(c, launch_scalar_fp64(c->g, sp, args, n, c->stream));
         }
     }
     if (host) {
@@ -1329,7 +1335,7 @@ int adjoint_core(mimadv_ctx *c, int integrator, int nsteps, double dt, const dou
                 a.c0 = s == 1 ? 0.0 : (s == 2 ? 0.75 : 1.0 / 3.0);
                 a.c1 = s == 1 ? 1.0 : (s == 2 ? 0.25 : 2.0 / 3.0);
             }
-            hipError_t e = launch_scalar_fp64(c->g, sp, a, c->stream);
+            hipError_t e = launch_scalar_fp64(c->g, sp, &a, 1, c->stream);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;

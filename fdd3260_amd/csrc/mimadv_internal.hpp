@@ -41,6 +41,31 @@ struct ScalarArgs {
     int fill;  // write periodic ghost images of every interior value (stage epilogues)
 };
 
+// Fields of one launch of a scalar operator (one per blockIdx.y): what they
+// share, and each one's arrays and form.
+constexpr int SCALAR_FIELDS = 8;
+struct ScalarList {
+    ScalarArgs all;
+    struct {
+        const double *q, *q0;
+        double *xs, *tend, *qn;
+        int adv;
+    } f[SCALAR_FIELDS];
+
+    void set(int n, const ScalarArgs &a) { f[n] = {a.q, a.q0, a.xs, a.tend, a.qn, a.adv}; }
+    __device__ __forceinline__ ScalarArgs field(int n) const
+    {
+        ScalarArgs a = all;
+        a.q = f[n].q;
+        a.q0 = f[n].q0;
+        a.xs = f[n].xs;
+        a.tend = f[n].tend;
+        a.qn = f[n].qn;
+        a.adv = f[n].adv;
+        return a;
+    }
+};
+
 // Adjoint of one Shu-Osher stage of the 'weno' flux-form tendency (adjoint.hip):
 //   out (=|+=) ic*qbn + (dL/dq)^T (ls*qbn);  acc0 (=|+=) c0*qbn;
 //   ub/vb/wb += (dL/d(u,v,w))^T (ls*qbn).  Interior cells only.
@@ -92,7 +117,10 @@ inline int levels_per_item(int nz, long tiles, int per_cu, int most)
 hipError_t launch_adjoint_stage(const AdjArgs &a, hipStream_t s);
 // dst = src on interior cells, 0 on ghost cells
 hipError_t launch_interior_copy(const GridDev &g, const double *src, double *dst, hipStream_t s);
-hipError_t launch_scalar_fp64(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s);
+// nf fields of one call (the arguments differ in q, q0, xs, tend, qn and adv
+// alone): in launches of up to SCALAR_FIELDS, fewer where arrays of the list
+// overlap, with the results of one launch per field.
+hipError_t launch_scalar_fp64(const GridDev &g, const SchemeParams &sp, const ScalarArgs *a, int nf, hipStream_t s);
 
 // One positivity-preserving Shu-Osher stage of the flux-form 'weno'
 // tendency: qn = c0*q0 + c1*(q + dt*L~(q)), L~ from face fluxes scaled by
@@ -106,7 +134,7 @@ struct PosArgs {
 hipError_t launch_positive_stage(const GridDev &g, const SchemeParams &sp, const PosArgs &a, hipStream_t s);
 // column-marching kernels (weno_march.hip): 'weno', WENO5, MUSCL, QUICK,
 // Lax-Wendroff and the unlimited forms
-hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s);
+hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, hipStream_t s);
 hipError_t launch_momentum_fp64(const GridDev &g, int mom_ord, int lavisc, int ntime, const double *mu,
                                 const double *mv, const double *mw, const double *ut, const double *vt,
                                 const double *wt, double *ua, double *va, double *wa, hipStream_t s);

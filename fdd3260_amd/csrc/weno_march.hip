@@ -484,40 +484,40 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
 // 256x256x128; WENO5 took 170 (2 waves).
 template <int TX, int TY>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) void weno_march_kernel(
-    GridDev g, SchemeParams sp, ScalarArgs a, int kchunk, int ntx, int nwork)
+    GridDev g, SchemeParams sp, ScalarList l, int kchunk, int ntx, int nwork)
 {
-    march_body<TX, TY, 0>(g, sp, a, kchunk, ntx, nwork);
+    march_body<TX, TY, 0>(g, sp, l.field(blockIdx.y), kchunk, ntx, nwork);
 }
 
 template <int TX, int TY>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) void weno5_march_kernel(
-    GridDev g, SchemeParams sp, ScalarArgs a, int kchunk, int ntx, int nwork)
+    GridDev g, SchemeParams sp, ScalarList l, int kchunk, int ntx, int nwork)
 {
-    march_body<TX, TY, 3>(g, sp, a, kchunk, ntx, nwork);
+    march_body<TX, TY, 3>(g, sp, l.field(blockIdx.y), kchunk, ntx, nwork);
 }
 
 template <int S, int TX, int TY>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) void line_march_kernel(
-    GridDev g, SchemeParams sp, ScalarArgs a, int kchunk, int ntx, int nwork)
+    GridDev g, SchemeParams sp, ScalarList l, int kchunk, int ntx, int nwork)
 {
-    march_body<TX, TY, S>(g, sp, a, kchunk, ntx, nwork);
+    march_body<TX, TY, S>(g, sp, l.field(blockIdx.y), kchunk, ntx, nwork);
 }
 
 template <int TX, int TY, int S>
-hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, int kchunk, hipStream_t s)
+hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, int kchunk, hipStream_t s)
 {
     const int ntx = (g.nx - 5 + TX - 1) / TX;
     const int nty = TY > 1 ? (g.ny - 5 + TY - 1) / TY : 1;
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
     const int nwork = ntx * nty * nchunk;
     if constexpr (S == 3)
-        hipLaunchKernelGGL((weno5_march_kernel<TX, TY>), dim3(nwork), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx,
+        hipLaunchKernelGGL((weno5_march_kernel<TX, TY>), dim3(nwork, nf), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx,
                            nwork);
     else if constexpr (S == 0)
-        hipLaunchKernelGGL((weno_march_kernel<TX, TY>), dim3(nwork), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx,
+        hipLaunchKernelGGL((weno_march_kernel<TX, TY>), dim3(nwork, nf), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx,
                            nwork);
     else
-        hipLaunchKernelGGL((line_march_kernel<S, TX, TY>), dim3(nwork), dim3(TX * TY), 0, s, g, sp, a, kchunk,
+        hipLaunchKernelGGL((line_march_kernel<S, TX, TY>), dim3(nwork, nf), dim3(TX * TY), 0, s, g, sp, a, kchunk,
                            ntx, nwork);
     return hipGetLastError();
 }
@@ -538,13 +538,13 @@ hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarArg
 // before; one round takes 68).  2D tiles are one wave each, 16 per CU: 38 -> 7
 // us at 128x128 (1 level; 16 before).
 template <int S, int TX3, int TY3>
-hipError_t launch_dims(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
+hipError_t launch_dims(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, hipStream_t s)
 {
     constexpr int MOST = 8;
     const long ntx3 = (g.nx - 5 + TX3 - 1) / TX3, nty3 = (g.ny - 5 + TY3 - 1) / TY3;
     if (g.ny > 1)
-        return launch_tile<TX3, TY3, S>(g, sp, a, levels_per_item(g.nz, ntx3 * nty3, S == 3 ? 8 : 4, MOST), s);
-    return launch_tile<64, 1, S>(g, sp, a, levels_per_item(g.nz, (g.nx - 5 + 63) / 64, 16, MOST), s);
+        return launch_tile<TX3, TY3, S>(g, sp, a, nf, levels_per_item(g.nz, ntx3 * nty3 * nf, S == 3 ? 8 : 4, MOST), s);
+    return launch_tile<64, 1, S>(g, sp, a, nf, levels_per_item(g.nz, (g.nx - 5 + 63) / 64 * nf, 16, MOST), s);
 }
 
 }  // namespace
@@ -679,16 +679,16 @@ hipError_t launch_positive_stage(const GridDev &g, const SchemeParams &sp, const
     return hipGetLastError();
 }
 
-hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarArgs &a, hipStream_t s)
+hipError_t launch_march(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, hipStream_t s)
 {
     switch (sp.scheme) {
-    case 0: return launch_dims<0, 32, 8>(g, sp, a, s);
-    case 3: return launch_dims<3, 16, 16>(g, sp, a, s);
-    case 2: return launch_dims<2, 32, 8>(g, sp, a, s);
-    case 4: return launch_dims<4, 32, 8>(g, sp, a, s);
-    case 5: return launch_dims<5, 32, 8>(g, sp, a, s);
-    case 6: return launch_dims<6, 32, 8>(g, sp, a, s);
-    case 7: return launch_dims<7, 32, 8>(g, sp, a, s);
+    case 0: return launch_dims<0, 32, 8>(g, sp, a, nf, s);
+    case 3: return launch_dims<3, 16, 16>(g, sp, a, nf, s);
+    case 2: return launch_dims<2, 32, 8>(g, sp, a, nf, s);
+    case 4: return launch_dims<4, 32, 8>(g, sp, a, nf, s);
+    case 5: return launch_dims<5, 32, 8>(g, sp, a, nf, s);
+    case 6: return launch_dims<6, 32, 8>(g, sp, a, nf, s);
+    case 7: return launch_dims<7, 32, 8>(g, sp, a, nf, s);
     default: return hipErrorInvalidValue;
     }
 }

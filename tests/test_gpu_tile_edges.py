@@ -270,3 +270,37 @@ def test_totalav_sizes(cuda, dims):
     assert abs(mean - float(inner.mean())) <= tol * mean
     want = float((inner.reshape(nz, -1).sum(axis=1) * np.asarray(g.dzw, dtype=np.longdouble)).sum())
     assert abs(budget - want) <= tol * want
+
+
+@pytest.mark.parametrize("scheme", ["weno", "weno5", "muscl", "ppm", "quick"])
+@pytest.mark.parametrize("dims", [(6, 6, 8), (45, 33, 20), (70, 0, 33)])
+@pytest.mark.parametrize("overlap", [False, True])
+def test_scalar_list_is_its_fields(cuda, scheme, dims, overlap):
+    """A list of fields, longer than a launch takes, of both forms, has the bits
+    of one call per field; so has one with a tendency that two fields add to
+    and one that is a later field's input."""
+    print(f"case scalar_list {scheme} {dims} overlap={overlap}", flush=True)
+    mx, my, nz = dims
+    g, u, v, w, _ = case3d(mx, my, nz) if my else case2d(mx, nz)
+    rng = np.random.default_rng(6)
+    n = 11
+    arrays = [1.0 + rng.random(g.shape) for _ in range(2 * n)]
+    form = [k % 2 for k in range(n)]
+    with Advection(g, scal_adv=scheme, muscllimiter="MC") as a:
+        vel = _dev(cuda, u, v, w)
+
+        def run(split):
+            d = _dev(cuda, *arrays)
+            q, xs = d[:n], d[n:]
+            if overlap:
+                xs[5] = xs[2]
+                xs[6] = q[7]
+            if split:
+                for f in range(n):
+                    a.scalar_tendency(0.5, *vel, [q[f]], [xs[f]], adv=[form[f]])
+            else:
+                a.scalar_tendency(0.5, *vel, q, xs, adv=form)
+            a.stream_sync()
+            return d
+        for k, (x, y) in enumerate(zip(run(False), run(True))):
+            assert torch.equal(x, y), f"array {k}"
