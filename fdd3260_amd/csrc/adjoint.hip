@@ -30,8 +30,9 @@
 //
 // Work mapping: a workgroup owns a TX x TY column tile and a chunk of
 // levels and marches up it.  Per level the x and y faces that touch the
-// tile (TX+3 per row, TY+3 per column) are evaluated once each and their
-// four stencil contributions are gathered through LDS; the z face k+1/2 is
+// tile (TX+3 per row, TY+3 per column) are evaluated once each, every thread
+// taking its cell's east and north face and some one of the left-over ones,
+// and their four stencil contributions are gathered through LDS; the z face k+1/2 is
 // evaluated by its column's thread and scattered into a register window of
 // the partial adjoints of levels k-1..k+2, level k-1 being complete after
 // it.  A chunk starts two levels early and ends one level late (z faces
@@ -212,9 +213,41 @@ __device__ __forceinline__ int perio(int i, int n, int m)
     return (r < 0 ? r + m : r) + 4;
 }
 
+// A lane's entry H of the halo of a TX x TY tile, HL cells wide and without its
+// corners: rows below, rows above, then the cells left and right of each row.
+// Row and column relative to the tile's first cell; false past the halo.
+template <int TX, int TY, int HL>
+__device__ __forceinline__ bool halo_cell(int h, int &r, int &c)
+{
+    constexpr int ROWS = TY > 1 ? HL * TX : 0;
+    if (h < 2 * ROWS) {
+        r = h / TX;
+        c = h - r * TX;
+        r = r < HL ? r - HL : r - HL + TY;
+        return true;
+    }
+    h -= 2 * ROWS;
+    if (h >= TY * 2 * HL) return false;
+    r = h / (2 * HL);
+    c = h - r * 2 * HL;
+    c = c < HL ? c - HL : c - HL + TX;
+    return true;
+}
+
 // S5: the WENO5-JS extension (6-cell face stencils q(f-2..f+3) in x and y,
 // in z where the upwind stencil lies in the column); otherwise the
 // reference 'weno' (4-cell stencils q(f-1..f+2)).
+//
+// Bound by HBM for 'weno': a stage at 256x256x128 reads q, qbn, u, v, w and
+// reads and writes ub, vb, wb, out and acc0, about 0.9 GB, 190 us at the rate
+// of a large copy, and takes 235 us (295 us before: tile centres loaded again
+// beside the column window, faces in a list with x and y mixed in a wave and
+// divisions for their place, the z face's velocity adjoint loaded where it is
+// used, 7 spilled registers).  128 VGPRs, four waves per SIMD; what makes
+// them enough is one face at a time (settle) and the requests for the next
+// level and the column after the faces, before the barrier: requested earlier they
+// spill (8 values cost 0.6 of 4.9 ms over twelve stages).  WENO5 is bound by
+// its arithmetic.
 template <int TX, int TY, bool S5>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 : 4, 8))) void adjoint_kernel(
     AdjArgs A)
@@ -225,17 +258,21 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
     constexpr int QHL = S5 ? 5 : 3;         // q tile halo
     constexpr int LHL = S5 ? 3 : 2;         // lam tile halo
     constexpr int FO = S5 ? 3 : 2;          // first face of a row: i0 - FO (+1/2)
-    constexpr int QW = TX + 2 * QHL, QH = THREE_D ? TY + 2 * QHL : 1;
-    constexpr int LW = TX + 2 * LHL, LH = THREE_D ? TY + 2 * LHL : 1;
+    constexpr int QW = TX + 2 * QHL, QH = THREE_D ? TY + 2 * QHL : 1, QY = THREE_D ? QHL : 0;
+    constexpr int LW = TX + 2 * LHL, LH = THREE_D ? TY + 2 * LHL : 1, LY = THREE_D ? LHL : 0;
     constexpr int NFX = TX + NS - 1, NFY = THREE_D ? TY + NS - 1 : 0;  // faces per row / column
     constexpr int NXF = TY * NFX, NYF = NFY * TX, NF = NXF + NYF;
-    constexpr int QS = (QH * QW + NT - 1) / NT, LS = (LH * LW + NT - 1) / NT, FS = (NF + NT - 1) / NT;
-    __shared__ double qt[QH][QW];
-    __shared__ double lt[LH][LW];
+    // faces that are no cell's east or north face
+    constexpr int LOX = TY * (NS - 1), LO = LOX + (THREE_D ? (NS - 1) * TX : 0);
+    constexpr int HQ = (THREE_D ? 2 * QHL * TX : 0) + TY * 2 * QHL, HL = (THREE_D ? 2 * LHL * TX : 0) + TY * 2 * LHL;
+    constexpr int QS = (HQ + NT - 1) / NT;
+    static_assert(HL <= NT && LO <= NT, "one lam halo value and one left-over face per thread at most");
+    __shared__ double qt[QH * QW];
+    __shared__ double lt[LH * LW];
     __shared__ double cf[NS][NF];  // stencil contributions per face, slot-major
-    // plane offsets of this thread's tile values and face velocities, fixed
-    // for the work item: [q tile (QS) | lam tile (LS) | faces (FS)] x NT
-    __shared__ unsigned slots[(QS + LS + FS) * NT];
+    // fixed for the work item, by thread: plane offset and place of its halo
+    // values; velocity offset, q and lam places and number of its left-over face
+    __shared__ unsigned slots[(2 * QS + 2 + 4) * NT];
 
     const int nx = A.nx, ny = A.ny, nz = A.nz, mx = nx - 5, my = ny - 5;
     const auto dz1w = table(A.dz1w);
@@ -251,51 +288,43 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
         const int k0 = 1 + kc * A.kchunk, k1 = min(nz, k0 + A.kchunk - 1);
         const int i = i0 + tx, j = j0 + ty;
         const bool valid = i <= nx - 2 && (!THREE_D || j <= ny - 2);
-        const int ip = perio(i, nx, mx), jp = THREE_D ? perio(j, ny, my) : 1;
-        const size_t col = (size_t)(ip - 1) + (size_t)nx * (jp - 1);
+        const auto at = [&](int ii, int jj) {
+            return (unsigned)((perio(ii, nx, mx) - 1) + nx * (THREE_D ? perio(jj, ny, my) - 1 : 0));
+        };
+        const unsigned col = at(i, j);
+        // velocity offsets of the east and north faces of this thread's cell
+        const unsigned east = at(i + 1, j), north = at(i, j + 1);
+        const auto slot = [&](int s) -> unsigned & { return slots[s * NT + tid]; };
 #pragma unroll
-        for (int s = 0; s < QS; ++s) {
-            const int t = tid + s * NT;
-            unsigned off = 0;
-            if (t < QH * QW) {
-                const int r = t / QW, c = t - r * QW;
-                const int ii = perio(i0 - QHL + c, nx, mx), jj = THREE_D ? perio(j0 - QHL + r, ny, my) : 1;
-                off = (unsigned)((ii - 1) + nx * (jj - 1));
-            }
-            slots[s * NT + tid] = off;
+        for (int s = 0; s <= QS; ++s) {
+            int r, c;
+            if (s < QS) {
+                if (halo_cell<TX, TY, QHL>(tid + s * NT, r, c)) {
+                    slot(2 * s) = at(i0 + c, j0 + r);
+                    slot(2 * s + 1) = (r + QY) * QW + c + QHL;
+                } else slot(2 * s) = col;
+            } else if (halo_cell<TX, TY, LHL>(tid, r, c)) {
+                slot(2 * s) = at(i0 + c, j0 + r);
+                slot(2 * s + 1) = (r + LY) * LW + c + LHL;
+            } else slot(2 * s) = col;
         }
-#pragma unroll
-        for (int s = 0; s < LS; ++s) {
-            const int t = tid + s * NT;
-            unsigned off = 0;
-            if (t < LH * LW) {
-                const int r = t / LW, c = t - r * LW;
-                const int ii = perio(i0 - LHL + c, nx, mx), jj = THREE_D ? perio(j0 - LHL + r, ny, my) : 1;
-                off = (unsigned)((ii - 1) + nx * (jj - 1));
-            }
-            slots[(QS + s) * NT + tid] = off;
+        constexpr int SF = 2 * QS + 2;
+        slot(SF) = col;
+        if (tid < LOX) {
+            // x face f + 1/2 (velocity u(f+1)), f = i0-FO+fl, of tile row r
+            const int r = tid / (NS - 1), n = tid - r * (NS - 1), fl = n < FO ? n : n + TX;
+            slot(SF) = at(i0 - FO + fl + 1, j0 + r);
+            slot(SF + 1) = (r + QY) * QW + fl;
+            slot(SF + 2) = (r + LY) * LW + fl;
+            slot(SF + 3) = r * NFX + fl;
+        } else if (tid < LO) {
+            // y face g + 1/2 (velocity v(g+1)), g = j0-FO+fr, of tile column c
+            const int n = (tid - LOX) / TX, c = tid - LOX - n * TX, fr = n < FO ? n : n + TY;
+            slot(SF) = at(i0 + c, j0 - FO + fr + 1);
+            slot(SF + 1) = fr * QW + c + QHL;
+            slot(SF + 2) = fr * LW + c + LHL;
+            slot(SF + 3) = NXF + fr * TX + c;
         }
-#pragma unroll
-        for (int s = 0; s < FS; ++s) {
-            const int e = tid + s * NT;
-            unsigned off = 0;
-            if (!THREE_D || e < NXF) {
-                if (e < NXF) {
-                    // x face f + 1/2 (velocity u(f+1)), f = i0-FO+fl, of tile row r
-                    const int r = e / NFX, fl = e - r * NFX, f = i0 - FO + fl;
-                    const int jr = THREE_D ? perio(j0 + r, ny, my) : 1;
-                    off = (unsigned)((perio(f + 1, nx, mx) - 1) + nx * (jr - 1));
-                }
-            } else if (e < NF) {
-                // y face g + 1/2 (velocity v(g+1)), g = j0-FO+fr, of tile column c
-                const int e2 = e - NXF, fr = e2 / TX, c = e2 - fr * TX, g = j0 - FO + fr;
-                off = (unsigned)((perio(i0 + c, nx, mx) - 1) + nx * (perio(g + 1, ny, my) - 1));
-            }
-            slots[(QS + LS + s) * NT + tid] = off;
-        }
-        auto q_off = [&](int s) { return slots[s * NT + tid]; };
-        auto l_off = [&](int s) { return slots[(QS + s) * NT + tid]; };
-        auto f_off = [&](int s) { return slots[(QS + LS + s) * NT + tid]; };
 
         // partial adjoints of levels k-ZL .. k-ZL+NS-1 (the levels the z
         // face k+1/2 touches)
@@ -305,128 +334,103 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
         for (int m = 0; m < NS; ++m) acc[m] = 0.0;
         auto finalize = [&](int m, double val, double qb) {
             if (!valid || m < k0 || m > k1) return;
-            const size_t id = col + (size_t)(m - 1) * plane;
+            const size_t km = (size_t)(m - 1) * plane;
+            double *out = A.out + km, *acc0 = A.acc0 + km;
             const double o = A.ic * qb + val;
-            if (A.accumulate) A.out[id] += o;
-            else A.out[id] = o;
-            if (A.acc0_mode == 1) A.acc0[id] = A.c0 * qb;
-            else if (A.acc0_mode == 2) A.acc0[id] += A.c0 * qb;
+            if (A.accumulate) out[col] += o;
+            else out[col] = o;
+            if (A.acc0_mode == 1) acc0[col] = A.c0 * qb;
+            else if (A.acc0_mode == 2) acc0[col] += A.c0 * qb;
         };
         // z faces f touching the chunk's levels: k0-NS/2 <= f <= k1+NS/2-1
         const int ks = max(1, k0 - NS / 2), ke = min(nz, k1 + NS / 2 - 1);
         // column values at level kk (clamped to 1..nz; q(0) := q(1) is the
         // floor convention of the first face)
-        auto Qz = [&](int kk) { return A.q[col + (size_t)(min(max(kk, 1), nz) - 1) * plane]; };
-        auto QBz = [&](int kk) { return A.qbn[col + (size_t)(min(max(kk, 1), nz) - 1) * plane]; };
+        auto level = [&](int kk) { return (size_t)(min(max(kk, 1), nz) - 1) * plane; };
+        auto Qz = [&](int kk) { return (A.q + level(kk))[col]; };
+        auto QBz = [&](int kk) { return (A.qbn + level(kk))[col]; };
         // register windows of iteration k: q(k-ZL..k-ZL+NS-1), qbn(k-ZL..k+1), w(k+1)
         double zq[NS], qbw[ZL + 2];
 #pragma unroll
         for (int m = 0; m < NS; ++m) zq[m] = Qz(ks - ZL + m);
 #pragma unroll
         for (int m = 0; m < ZL + 2; ++m) qbw[m] = QBz(ks - ZL + m);
-        double wz = ks <= nz - 1 ? A.w[col + (size_t)ks * plane] : 0.0;
-        // tile values and face velocities of a chunk level, requested one
-        // level ahead
-        double qv[QS], lv[LS], fv[FS];
+        double wz = (A.w + level(ks + 1))[col];
+        // halo values and face velocities of a chunk level, requested one
+        // level ahead; threads without one load an address of their own column
+        double qh[QS], lh, ue, vn = 0.0, vl;
         auto fetch = [&](int k) {
             const size_t kb = (size_t)(k - 1) * plane;
             const double *qk = A.q + kb, *lk = A.qbn + kb, *uk = A.u + kb, *vk = A.v + kb;
 #pragma unroll
-            for (int s = 0; s < QS; ++s)
-                if (tid + s * NT < QH * QW) qv[s] = qk[q_off(s)];
+            for (int s = 0; s < QS; ++s) qh[s] = qk[slot(2 * s)];
+            lh = lk[slot(2 * QS)];
+            ue = uk[east];
+            if constexpr (THREE_D) vn = vk[north];
+            vl = (!THREE_D || tid < LOX ? uk : vk)[slot(SF)];
+        };
+        // R of a face from q at qb, qb + st, ... and its four contributions
+        auto face = [&](const double *qb, int st, double uf, double Fb, double *gs) {
 #pragma unroll
-            for (int s = 0; s < LS; ++s)
-                if (tid + s * NT < LH * LW) lv[s] = lk[l_off(s)];
+            for (int m = 0; m < NS; ++m) gs[m] = 0.0;
+            if constexpr (S5) {
+                double sv[NS];
 #pragma unroll
-            for (int s = 0; s < FS; ++s) {
-                const int e = tid + s * NT;
-                fv[s] = (!THREE_D || e < NXF) ? (e < NXF ? uk[f_off(s)] : 0.0) : (e < NF ? vk[f_off(s)] : 0.0);
+                for (int m = 0; m < NS; ++m) sv[m] = qb[m * st];
+                return face5_vjp(sv, !(uf < 0.0), Fb * uf, gs);
+            } else {
+                return face_vjp(qb[0], qb[st], qb[2 * st], qb[3 * st], !(uf < 0.0), 0, true, Fb * uf, gs[0], gs[1],
+                                gs[2], gs[3]);
             }
         };
         fetch(k0);
 #pragma unroll 1
         for (int k = ks; k <= ke; ++k) {
             const size_t kb = (size_t)(k - 1) * plane;
-            // the next iteration's column values, requested now
-            double zn = 0.0, qbn1 = 0.0, wn = 0.0;
-            if (k < ke) {
-                zn = Qz(k + NS - ZL);
-                qbn1 = QBz(k + 2);
-                wn = k + 1 <= nz - 1 ? A.w[col + (size_t)(k + 1) * plane] : 0.0;
-            }
             if (k >= k0 && k <= k1) {
+                qt[(ty + QY) * QW + tx + QHL] = zq[ZL];
+                const double lam = A.ls * qbw[ZL];
+                lt[(ty + LY) * LW + tx + LHL] = lam;
 #pragma unroll
                 for (int s = 0; s < QS; ++s)
-                    if (tid + s * NT < QH * QW) (&qt[0][0])[tid + s * NT] = qv[s];
-#pragma unroll
-                for (int s = 0; s < LS; ++s)
-                    if (tid + s * NT < LH * LW) (&lt[0][0])[tid + s * NT] = A.ls * lv[s];
-                double vc[FS];
-#pragma unroll
-                for (int s = 0; s < FS; ++s) vc[s] = fv[s];
+                    if (tid + s * NT < HQ) qt[slot(2 * s + 1)] = qh[s];
+                if (tid < HL) lt[slot(2 * QS + 1)] = A.ls * lh;
+                const double uf = ue, vf = vn, lf = vl;
                 __syncthreads();
-                if (k < k1) fetch(k + 1);
-                // the velocity adjoints of the faces this thread owns, requested
-                // before the face arithmetic that updates them
-                double vbo[FS];
-                bool own[FS];
+                // the velocity adjoints this thread updates, requested before the
+                // face arithmetic
+                const double ubo = (A.ub + kb)[east];
+                double vbo = 0.0;
+                if constexpr (THREE_D) vbo = (A.vb + kb)[north];
+                double gs[NS];
+                {
+                    const double Fb = (lt[(ty + LY) * LW + tx + LHL + 1] - lam) * A.dx1;
+                    const double R = face(&qt[(ty + QY) * QW + tx + FO], 1, uf, Fb, gs);
+                    if (valid) (A.ub + kb)[east] = ubo + Fb * R;
 #pragma unroll
-                for (int s = 0; s < FS; ++s) {
-                    const int e = tid + s * NT;
-                    own[s] = false;
-                    vbo[s] = 0.0;
-                    if (e >= NF) continue;
-                    if (!THREE_D || e < NXF) {
-                        const int r = e / NFX, f = i0 - FO + (e - r * NFX);
-                        own[s] = f >= i0 && f < i0 + TX && f <= nx - 2 && (!THREE_D || j0 + r <= ny - 2);
-                        if (own[s]) vbo[s] = A.ub[kb + f_off(s)];
-                    } else {
-                        const int e2 = e - NXF, fr = e2 / TX, c = e2 - fr * TX, g = j0 - FO + fr;
-                        own[s] = g >= j0 && g < j0 + TY && g <= ny - 2 && i0 + c <= nx - 2;
-                        if (own[s]) vbo[s] = A.vb[kb + f_off(s)];
+                    for (int m = 0; m < NS; ++m) {
+                        settle(gs[m]);
+                        cf[m][ty * NFX + tx + FO] = gs[m];
                     }
                 }
+                if constexpr (THREE_D) {
+                    const double Fb = (lt[(ty + LY + 1) * LW + tx + LHL] - lam) * A.dy1;
+                    double fv = vf;
+                    settle(fv);
+                    const double R = face(&qt[(ty + FO) * QW + tx + QHL], QW, fv, Fb, gs);
+                    if (valid) (A.vb + kb)[north] = vbo + Fb * R;
 #pragma unroll
-                for (int s = 0; s < FS; ++s) {
-                    const int e = tid + s * NT;
-                    if (e >= NF) continue;
-                    double gs[NS];
-#pragma unroll
-                    for (int m = 0; m < NS; ++m) gs[m] = 0.0;
-                    if (!THREE_D || e < NXF) {
-                        // x face f + 1/2 (velocity u(f+1)), f = i0-FO+fl, of tile row r
-                        const int r = e / NFX, fl = e - r * NFX;
-                        const double uf = vc[s];
-                        const int lr = THREE_D ? r + LHL : 0, qr = THREE_D ? r + QHL : 0;
-                        const double Fb = (lt[lr][fl + 1] - lt[lr][fl]) * A.dx1;
-                        double R;
-                        if constexpr (S5) {
-                            double sv[NS];
-#pragma unroll
-                            for (int m = 0; m < NS; ++m) sv[m] = qt[qr][fl + m];
-                            R = face5_vjp(sv, !(uf < 0.0), Fb * uf, gs);
-                        } else {
-                            R = face_vjp(qt[qr][fl], qt[qr][fl + 1], qt[qr][fl + 2], qt[qr][fl + 3], !(uf < 0.0), 0,
-                                         true, Fb * uf, gs[0], gs[1], gs[2], gs[3]);
-                        }
-                        if (own[s]) A.ub[kb + f_off(s)] = vbo[s] + Fb * R;
-                    } else if constexpr (THREE_D) {
-                        // y face g + 1/2 (velocity v(g+1)), g = j0-FO+fr, of tile column c
-                        const int e2 = e - NXF, fr = e2 / TX, c = e2 - fr * TX;
-                        const double vf = vc[s];
-                        const double Fb = (lt[fr + 1][c + LHL] - lt[fr][c + LHL]) * A.dy1;
-                        double R;
-                        if constexpr (S5) {
-                            double sv[NS];
-#pragma unroll
-                            for (int m = 0; m < NS; ++m) sv[m] = qt[fr + m][c + QHL];
-                            R = face5_vjp(sv, !(vf < 0.0), Fb * vf, gs);
-                        } else {
-                            R = face_vjp(qt[fr][c + 3], qt[fr + 1][c + 3], qt[fr + 2][c + 3], qt[fr + 3][c + 3],
-                                         !(vf < 0.0), 0, true, Fb * vf, gs[0], gs[1], gs[2], gs[3]);
-                        }
-                        if (own[s]) A.vb[kb + f_off(s)] = vbo[s] + Fb * R;
+                    for (int m = 0; m < NS; ++m) {
+                        settle(gs[m]);
+                        cf[m][NXF + (ty + FO) * TX + tx] = gs[m];
                     }
+                }
+                fetch(min(k + 1, k1));
+                if (tid < LO) {
+                    const bool x = !THREE_D || tid < LOX;
+                    const unsigned ql = slot(SF + 1), ll = slot(SF + 2), e = slot(SF + 3);
+                    const double Fb = (lt[ll + (x ? 1 : LW)] - lt[ll]) * (x ? A.dx1 : A.dy1);
+                    face(&qt[ql], x ? 1 : QW, lf, Fb, gs);
 #pragma unroll
                     for (int m = 0; m < NS; ++m) cf[m][e] = gs[m];
                 }
@@ -447,6 +451,10 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
                 // and cf is rewritten only after the next level's first
                 // barrier, which every thread reaches after its gather
             }
+            // the next iteration's column values and the adjoint of w(k+1), wanted
+            // after the z face
+            const double zn = Qz(k + NS - ZL), qbn1 = QBz(k + 2), wn = (A.w + level(k + 2))[col];
+            const double wbo = (A.wb + level(k + 1))[col];
             // z face k+1/2 (velocity w(k+1)); no flux through floor and lid
             if (k <= nz - 1) {
                 const double Fb = A.ls * (qbw[ZL + 1] * dz1w[k] - qbw[ZL] * dz1w[k - 1]);
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
                     acc[ZL + 1] += gc;
                     acc[ZL + 2] += gd;
                 }
-                if (valid && k >= k0 && k <= k1) A.wb[col + (size_t)k * plane] += Fb * R;
+                if (valid && k >= k0 && k <= k1) (A.wb + (size_t)k * plane)[col] = wbo + Fb * R;
             }
             finalize(k - ZL, acc[0], qbw[0]);
 #pragma unroll
@@ -501,10 +509,16 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(S5 ? 2 :
 }
 
 template <int TX, int TY, bool S5>
-hipError_t launch_tile(AdjArgs A, hipStream_t s)
+hipError_t launch_tile(AdjArgs A, int per_cu, hipStream_t s)
 {
     A.ntx = (A.nx - 5 + TX - 1) / TX;
     A.nty = TY > 1 ? (A.ny - 5 + TY - 1) / TY : 1;
+    // A chunk's z faces beyond its levels and its first loads measure like two
+    // levels.  Chunks of 16 levels -> this rule, two SSP-RK3 steps: 'weno'
+    // 24x24x16 334 -> 103 us, 96x96x48 411 -> 230, 139x117x75 503 -> 461,
+    // 192x160x96 876 -> 753; WENO5 560 -> 148, 675 -> 398, 1015 -> 820.
+    if (A.kchunk <= 0) A.kchunk = levels_by_rounds(A.nz, (long)A.ntx * A.nty, per_cu, 2);
+    A.kchunk = min(A.kchunk, A.nz);
     const int nchunk = (A.nz + A.kchunk - 1) / A.kchunk;
     A.nwork = A.ntx * A.nty * nchunk;
     hipLaunchKernelGGL((adjoint_kernel<TX, TY, S5>), dim3(A.nwork), dim3(TX * TY), 0, s, A);
@@ -530,20 +544,19 @@ hipError_t launch_interior_copy(const GridDev &g, const double *src, double *dst
     return hipGetLastError();
 }
 
-hipError_t launch_adjoint_stage(const AdjArgs &a0, hipStream_t s)
+hipError_t launch_adjoint_stage(const AdjArgs &a, hipStream_t s)
 {
-    AdjArgs A = a0;
-    if (A.kchunk <= 0) A.kchunk = 16;
-    if (A.kchunk > A.nz) A.kchunk = A.nz;
-    if (A.weno5) {
+    // groups per CU: 68 KB of LDS (64x8), three waves per SIMD (WENO5), four
+    if (a.weno5) {
         // 6-cell stencils: a 16x16 tile has the fewest faces per cell
-        // (672 for 256 cells), so its face contributions, tiles and slot
-        // offsets take 49.7 KB of LDS and three groups share a CU
-        if (A.ny > 1) return launch_tile<16, 16, true>(A, s);
-        return launch_tile<64, 1, true>(A, s);
+        // (672 for 256 cells), so its face contributions, tiles and slots
+        // take 51.8 KB of LDS and three groups share a CU
+        if (a.ny > 1) return launch_tile<16, 16, true>(a, 3, s);
+        return launch_tile<64, 1, true>(a, 12, s);
     }
-    if (A.ny > 1) return launch_tile<64, 8, false>(A, s);
-    return launch_tile<64, 1, false>(A, s);
+    // 32x16 tiles have 6 % fewer faces and take 1 % longer (half the row per load)
+    if (a.ny > 1) return launch_tile<64, 8, false>(a, 2, s);
+    return launch_tile<64, 1, false>(a, 16, s);
 }
 
 }  // namespace mimadv

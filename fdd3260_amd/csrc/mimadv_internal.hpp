@@ -113,6 +113,26 @@ inline int levels_per_item(int nz, long tiles, int per_cu, int most)
     return (int)std::min<long>(nz, std::max<long>(1, std::min<long>(most, levels)));
 }
 
+// Levels per work item where starting an item costs as much as `fill` levels:
+// items run in rounds of per_cu groups per CU, so the length with the least
+// rounds * (levels + fill) is taken, the longest of equals.  Small grids get
+// short items on all CUs, and tiles that fill a round and a part of one are
+// cut until the rounds are nearly full.
+inline int levels_by_rounds(int nz, long tiles, int per_cu, int fill)
+{
+    const long slots = (long)per_cu * device_cus();
+    int levels = nz;
+    long best = 0;
+    for (int k = nz; k >= 1; --k) {
+        const long rounds = (tiles * ((nz + k - 1) / k) + slots - 1) / slots;
+        if (best == 0 || rounds * (k + fill) < best) {
+            best = rounds * (k + fill);
+            levels = k;
+        }
+    }
+    return levels;
+}
+
 // Launchers (scalar_fp64.hip, momentum_fp64.hip, util.hip, adjoint.hip).
 hipError_t launch_adjoint_stage(const AdjArgs &a, hipStream_t s);
 // dst = src on interior cells, 0 on ghost cells

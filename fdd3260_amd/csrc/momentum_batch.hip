@@ -423,26 +423,12 @@ hipError_t launch_momentum_batch(const GridDev &g, int mom_ord, int lavisc, cons
     const bool three_d = g.ny > 1;
     const int ntx3 = (g.nx - 5 + 31) / 32, nty3 = (g.ny - 5 + 7) / 8;
     const int tiles = three_d ? ntx3 * nty3 : (g.nx - 5 + 63) / 64;
-    // Levels per work item: items run in rounds of four groups per CU (2D:
-    // sixteen), each taking as long as its levels and the ring fill, which
-    // measures like two more.  The length with the least rounds * (levels +
-    // fill) is taken, the longest of equals: a small grid marches one or two
-    // levels per item on all CUs, 1024 tiles march whole columns (4 % faster
-    // than 32-level items, which are 4 % faster than 16-level ones), and
-    // tiles that fill a round and a part of one are cut until the rounds are
-    // nearly full.  Tendencies of 20 fields, whole columns or at least 32
-    // levels -> this rule: 96x96x48 (36 tiles) 301 -> 196 us, 192x160x96 (120)
-    // 531 -> 468 us, 400x400x100 (650) 1142 -> 1049 us for 8 fields.
-    const long slots = (long)(three_d ? 4 : 16) * device_cus();
-    int kchunk = g.nz;
-    long best = 0;
-    for (int k = g.nz; k >= 1; --k) {
-        const long rounds = ((long)tiles * ((g.nz + k - 1) / k) + slots - 1) / slots;
-        if (best == 0 || rounds * (k + 2) < best) {
-            best = rounds * (k + 2);
-            kchunk = k;
-        }
-    }
+    // Four groups per CU (2D: sixteen); an item's ring fill measures like two
+    // levels.  1024 tiles march whole columns (4 % faster than 32-level items,
+    // which are 4 % faster than 16-level ones).  Whole columns or at least 32
+    // levels -> this rule: 20 fields at 96x96x48 (36 tiles) 301 -> 196 us, at
+    // 192x160x96 (120) 531 -> 468 us, 8 fields at 400x400x100 (650) 1121 -> 1049 us.
+    const int kchunk = levels_by_rounds(g.nz, tiles, three_d ? 4 : 16, 2);
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
     if (three_d) {
         constexpr int TX = 32, TY = 8;

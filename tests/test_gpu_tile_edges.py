@@ -9,6 +9,7 @@ from fdd3260_amd import Advection
 from oracle.oracle import Oracle
 
 from helpers import case2d, case3d
+from test_gpu_adjoint import _case as adjoint_case, _check_dot, _dirs, _interior_only, _mask, _tlm
 
 pytestmark = pytest.mark.gpu
 
@@ -304,3 +305,35 @@ def test_scalar_list_is_its_fields(cuda, scheme, dims, overlap):
             return d
         for k, (x, y) in enumerate(zip(run(False), run(True))):
             assert torch.equal(x, y), f"array {k}"
+
+
+@pytest.mark.parametrize("scheme", ["weno", "weno5"])
+@pytest.mark.parametrize("dims", [(6, 6, 8), (63, 7, 9), (64, 8, 33), (65, 9, 17), (17, 16, 10), (130, 33, 12),
+                                  (64, 0, 9), (65, 0, 20)])
+def test_adjoint_tile_edges(cuda, scheme, dims):
+    """<lam, L' d> = <L'^T lam, d> with the oracle's tangent one cell around the
+    tiles of both instances, to the 1e-13 of the other dot products; a second
+    call writes the same qbar and adds to the velocity adjoints again."""
+    print(f"case adjoint_edges {scheme} {dims}", flush=True)
+    mx, my, nz = dims
+    g, u, v, w, q = adjoint_case(my > 0, "gaussian", maxx=mx, maxy=my, nz=nz)
+    rng = np.random.default_rng(72)
+    dq, du, dv, dw = _dirs(g, rng, np.abs(q).mean())
+    lam = _interior_only(g, rng.standard_normal(g.shape))
+    _, tl = _tlm(Oracle(g, scal_adv=scheme), scheme)(q, dq, u, v, w, du, dv, dw)
+    with Advection(g, scal_adv=scheme) as a:
+        U, V, W, Q, L = _dev(cuda, u, v, w, q, lam)
+        bars = [torch.zeros_like(Q) for _ in range(4)]
+        a.adjoint_tendency(U, V, W, Q, L, *bars)
+        a.stream_sync()
+        once = [x.cpu().numpy() for x in bars]
+        a.adjoint_tendency(U, V, W, Q, L, *bars)
+        a.stream_sync()
+        twice = [x.cpu().numpy() for x in bars]
+    I = g.interior()
+    assert np.all(once[0][~_mask(g)] == 0.0), "ghost entries of qbar were written"
+    _check_dot([lam[I] * tl[I]], [d * x for d, x in zip((dq, du, dv, dw), once)])
+    assert np.array_equal(once[0], twice[0])
+    for n, (x, y) in enumerate(zip(once[1:], twice[1:])):
+        scale = max(float(np.abs(x).max()), 1e-300)
+        assert float(np.abs(y - 2.0 * x).max()) <= 4 * 2.0 ** -52 * scale, f"velocity {n}"
