@@ -388,6 +388,10 @@ hipError_t launch_scalar_fp64(const GridDev &g, const SchemeParams &sp, const Sc
     for (int f0 = 0; f0 < nf;) {
         ScalarList l = {};
         l.all = a[f0];
+        // a component that no direction of the call uses may be missing; the
+        // kernels load all of them
+        for (const double **c : {&l.all.u, &l.all.v, &l.all.w})
+            if (!*c) *c = a[f0].q;
         l.set(0, a[f0]);
         int n1 = 1;
         for (bool ok = true; ok && n1 < SCALAR_FIELDS && f0 + n1 < nf; n1 += ok) {

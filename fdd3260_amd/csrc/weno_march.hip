@@ -310,28 +310,24 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
         // WENO5 widens the window to q(k-2..k+3)
         double zm1 = S == 3 ? Qz(kstart - 2) : 0.0, z4 = S == 3 ? Qz(kstart + 3) : 0.0;
         double wz = kstart < nz ? a.w[col + (size_t)kstart * plane] : 0.0;
-        double fzb = 0.0;
-        // operands of level k, requested one level ahead
+        double fzb = 0.0, wb = 0.0;  // face below: flux and w
+        // operands of level k, requested one level ahead by every thread: a load
+        // under a lane mask ends in a wait for all outstanding ones (Heun step of
+        // two 'weno' fields at 256x256x128 620 -> 590 us, four MUSCL tendencies at
+        // 190x131x75 152 -> 140 us).  Empty slots and the last level load again.
         double tv[TS], vv[FS], wv = 0.0, zn = 0.0, q0v = 0.0, tdv = 0.0, xsv = 0.0;
         auto fetch = [&](int k) {
             const size_t kb = (size_t)(k - 1) * plane;
             const double *qk = a.q + kb, *uk = a.u + kb, *vk = a.v + kb;
 #pragma unroll
-            for (int s = 0; s < TS; ++s)
-                if (tid + s * NT < LH * LW) tv[s] = qk[t_off(s)];
+            for (int s = 0; s < TS; ++s) tv[s] = qk[t_off(s)];
 #pragma unroll
-            for (int s = 0; s < FS; ++s)
-            {
-                const int kind = f_slot(s) >> 16;
-                vv[s] = kind == 1 ? uk[f_off(s)] : (kind == 2 ? vk[f_off(s)] : 0.0);
-            }
-            wv = k < nz ? a.w[col + kb + plane] : 0.0;
+            for (int s = 0; s < FS; ++s) vv[s] = (f_slot(s) >> 16 == 2 ? vk : uk)[f_off(s)];
+            wv = a.w[col + (size_t)min(k, nz - 1) * plane];
             zn = Qz(S == 3 ? k + 3 : k + 2);
-            if (valid) {
-                if (need_q0) q0v = a.q0[col + kb];
-                if (need_tend) tdv = a.tend[col + kb];
-                if (accum) xsv = a.xs[col + kb];
-            }
+            if (need_q0) q0v = a.q0[col + kb];
+            if (need_tend) tdv = a.tend[col + kb];
+            if (accum) xsv = a.xs[col + kb];
         };
         fetch(k0);
 #pragma unroll 1
@@ -377,6 +373,7 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
             }
             if (k < k0) {
                 fzb = fzt;
+                wb = wc;
                 continue;
             }
             const size_t kb = (size_t)(k - 1) * plane;
@@ -387,7 +384,16 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
             for (int s = 0; s < FS; ++s) fvel[tid + s * NT] = vv[s];
             const double q0c = q0v, tdc = tdv, xsc = xsv;
             __syncthreads();
-            if (k < k1) fetch(k + 1);
+            fetch(min(k + 1, k1));
+            // velocity differences of the advective form, from the staged face
+            // velocities (WENO5 step at 139x117x75 366 -> 350 us: they were loaded
+            // where the cell uses them)
+            double du = 0.0, dv = 0.0;
+            if (adv) {
+                const int e = ty * (TX + 1) + tx, n = NXF + ty * TX + tx;
+                du = fvel[e + 1] - fvel[e];
+                if (THREE_D) dv = fvel[n + TX] - fvel[n];
+            }
             // one face at a time: the exact FP64 face is register-hungry
 #pragma unroll 1
             for (int s = 0; s < FS; ++s) {
@@ -404,24 +410,18 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
                 if (a.dirmask & 1) {
                     const int e = ty * (TX + 1) + tx;
                     X = (face[e + 1] - face[e]) * dx1;
-                    if (adv) {
-                        const double *urow = a.u + kb + (size_t)nx * (j - 1);
-                        X = X - z1 * (urow[i] - urow[i - 1]) * dx1;
-                    }
+                    if (adv) X = X - z1 * du * dx1;
                 }
                 if (THREE_D && (a.dirmask & 2)) {
                     const int e = NXF + ty * TX + tx;
                     Y = (face[e + TX] - face[e]) * dy1;
-                    if (adv) {
-                        const double *vcol = a.v + kb + (size_t)(i - 1);
-                        Y = Y - z1 * (vcol[(size_t)nx * j] - vcol[(size_t)nx * (j - 1)]) * dy1;
-                    }
+                    if (adv) Y = Y - z1 * dv * dy1;
                 }
                 if (zdir) {
                     // z_assemble (no-flux 'nnf' floor/lid, zero z tendency at other ends)
                     if (k >= 2 && k <= nz - 1) {
                         Z = (fzt - fzb) * dz1w[k - 1];
-                        if (adv) Z = Z - z1 * (wc - a.w[col + kb]) * dz1w[k - 1];
+                        if (adv) Z = Z - z1 * (wc - wb) * dz1w[k - 1];
                     } else {
                         double t = 0.0;
                         if (k == 1 && bc5 == 1) {
@@ -430,7 +430,7 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
                         }
                         if (k == nz && bc6 == 1) {
                             t = t + (0.0 - fzb) * dz1w[nz - 1];
-                            if (adv) t = t - z1 * (0.0 - a.w[col + kb]) * dz1w[nz - 1];
+                            if (adv) t = t - z1 * (0.0 - wb) * dz1w[nz - 1];
                         }
                         Z = t;
                     }
@@ -474,6 +474,7 @@ __device__ __forceinline__ void march_body(const GridDev &g, const SchemeParams 
                 }
             }
             fzb = fzt;
+            wb = wc;
         }
     }
 }
