@@ -8,12 +8,12 @@
 //   * the chunk's face velocities are staged in LDS once and serve every
 //     field of the batch (fields are the outer loop, levels the inner one,
 //     so register use does not grow with the field count);
-//   * per field and level the tile plus a 2-cell halo goes through LDS
-//     (the next level's tile is already in flight), the TY*(TX+1) x faces
-//     and (TY+1)*TX y faces of the tile are evaluated once each by a
-//     flattened loop over the workgroup, and the z face k+1/2 of every
-//     column comes from a register window q(k-1..k+2) and is carried to
-//     level k+1 as its bottom face;
+//   * per field and level the tile plus a 2-cell halo goes through LDS (a
+//     thread's own value from its column window, the halo requested a level
+//     ahead), every thread forms the west and south face of its cell, one
+//     wave the faces beyond the last column and row, and the z face k+1/2
+//     of every column comes from a register window q(k-1..k+2) and is
+//     carried to level k+1 as its bottom face;
 //   * face fluxes of FP32 fields are FP32; the flux differences and the
 //     divergence are accumulated in FP64 (exact differences of FP32 values,
 //     a compensated sum) and the Shu-Osher stage update
@@ -40,117 +40,83 @@ namespace {
 using namespace faces;
 
 // Geometry of one work item (a TX x TY column tile and a chunk of at most
-// KC levels) shared by every field it advects.
+// KC levels) shared by every field it advects.  A thread owns the cell (tx,
+// ty), its west face and its south face; the faces beyond the tile's last
+// column and row are `LO` left-over ones.
 template <int TX, int TY, int H>
 struct Item {
     static constexpr bool THREE_D = TY > 1;
     static constexpr int NT = TX * TY;
     static constexpr int LW = TX + 2 * H, LH = THREE_D ? TY + 2 * H : 1;  // tile + H-cell halo
-    static constexpr int NXF = TY * (TX + 1), NYF = THREE_D ? (TY + 1) * TX : 0, NF = NXF + NYF;
-    static constexpr int FS = (NF + NT - 1) / NT;        // face slots per thread
-    static constexpr int TS = (LH * LW + NT - 1) / NT;   // tile slots per thread
-    static constexpr int NV = NF + NT;                   // velocities per level: faces, then w of every column
+    static constexpr int LO = TY + (THREE_D ? TX : 0);                   // east faces, then north faces
+    static constexpr int NH = 2 * H * (TY + (THREE_D ? TX : 0));         // halo values (no corners)
+    static constexpr int HS = (NH + NT - 1) / NT;                        // halo slots per thread
+    static constexpr int NFACE = (THREE_D ? 2 * NT : NT) + LO;           // west, south, left-over
+    static constexpr int SOUTH = NT, REST = THREE_D ? 2 * NT : NT;       // their offsets
+    static constexpr int NV = NFACE + NT;                                // velocities per level: faces, then w
 };
 
 // Levels of a work item whose velocities are staged in LDS once and read by
 // every field (the chunk length is capped at this).
 constexpr int FUSED_KC = 8;
 
-// The FP32 256-thread tiles of the WENO and MUSCL schemes: six-level chunks
-// take 25 KB of LDS, so six groups of four waves fit a CU, and the kernel
-// is held to 80 VGPRs (a few values of the per-item velocity staging spill;
-// the level loop does not).  The FP64 and WENO5 instances are bound by
-// their registers and keep eight-level chunks.
-template <int SCHEME, int TX, int TY, class T>
-constexpr bool fused_six_waves()
-{
-    return SCHEME != 3 && TX * TY == 256 && TY > 1 && sizeof(T) == 4;
-}
+// The 256-thread tiles take shorter chunks: their LDS bounds how many groups
+// share a CU, and more groups hide more than the velocity staging of a longer
+// chunk saves.  FP32 six levels (23 KB, seven groups; WENO5 24 KB, six), FP64
+// five (24 KB, six groups).  A step of 20 fields at 512x512x160: 6 and 8
+// levels 15.54 ms, 6 and 5 15.44, 5 and 8 15.51, 4 and 8 15.65, 8 and 8 16.24;
+// ten WENO5 species with two FP64 fields at 256x256x128: 8 and 8 1.08 ms, 6 and 5 1.02.
 template <int SCHEME, int TX, int TY, class T>
 constexpr int fused_kc()
 {
-    return fused_six_waves<SCHEME, TX, TY, T>() ? 6 : FUSED_KC;
+    return TX * TY != 256 ? FUSED_KC : sizeof(T) == 8 ? 5 : 6;
 }
 
-// Face e of the flattened list [x faces row-major | y faces] of a tile:
-// kind (1 x, 2 y), LDS offset/step of its stencil and the column of its
-// velocity (u(f+1) of x face f + 1/2, v(g+1) of y face g + 1/2).
+// This thread's part of the halo of a work item's tile, the same for every
+// field and level: offsets in a level plane (32 bits; threads past the end of the list
+// load their own column) and in the LDS tile.  The list holds the H columns west and east of
+// every row, then the H rows south and north of every column; no face reads a
+// corner.
 template <int TX, int TY, int H>
-__device__ __forceinline__ int face_slot_geom(int e, int i0, int j0, const FusedArgs &A, int &base, int &step,
-                                              size_t &vcol)
-{
+struct Halo {
     using I = Item<TX, TY, H>;
-    const int nx = A.nx, ny = A.ny;
-    if (e < I::NXF) {
-        const int r = e / (TX + 1), fl = e - r * (TX + 1);
-        base = (I::THREE_D ? r + H : 0) * I::LW + fl;
-        step = 1;
-        const int jr = I::THREE_D ? wrap(j0 + r, ny, A.my) : 1;
-        vcol = (size_t)(wrap(i0 + fl, nx, A.mx) - 1) + (size_t)nx * (jr - 1);
-        return 1;
-    }
-    const int e2 = e - I::NXF, fr = e2 / TX, c = e2 - fr * TX;
-    base = fr * I::LW + c + H;
-    step = I::LW;
-    vcol = (size_t)(wrap(i0 + c, nx, A.mx) - 1) + (size_t)nx * (wrap(j0 + fr, ny, A.my) - 1);
-    return 2;
-}
-
-// Per-thread slot geometry of a work item, computed once and shared by
-// every field and level: the thread's tile slots (column offset in a level
-// plane, -1 if none) and face slots of the flattened list
-// [x faces row-major | y faces] (LDS offset of the stencil q(f-1..f+2),
-// step 1 for x and LW for y, 0 for an empty slot).  Plane offsets fit in
-// 32 bits.
-template <int TX, int TY, int H>
-struct Slots {
-    using I = Item<TX, TY, H>;
-    int t_off[I::TS];
-    int f_base[I::FS], f_step[I::FS];
+    int off[I::HS], pos[I::HS];
     __device__ __forceinline__ void init(int tid, int i0, int j0, const FusedArgs &A)
     {
-        const int nx = A.nx, ny = A.ny;
 #pragma unroll
-        for (int s = 0; s < I::TS; ++s) {
-            const int e = tid + s * I::NT;
-            t_off[s] = -1;
-            if (e < I::LH * I::LW) {
-                const int r = e / I::LW, c = e - r * I::LW;
-                const int ii = wrap(i0 - H + c, nx, A.mx);
-                const int jj = I::THREE_D ? wrap(j0 - H + r, ny, A.my) : 1;
-                t_off[s] = (ii - 1) + nx * (jj - 1);
+        for (int s = 0; s < I::HS; ++s) {
+            const int e = tid + s * I::NT, el = min(e, I::NH - 1);
+            int r, c;
+            if (el < 2 * H * TY) {
+                r = el / (2 * H) + (I::THREE_D ? H : 0);
+                c = el % (2 * H);
+                c = c < H ? c : c + TX;
+            } else {
+                const int e2 = el - 2 * H * TY;
+                r = e2 / TX;
+                r = r < H ? r : r + TY;
+                c = e2 % TX + H;
             }
-        }
-#pragma unroll
-        for (int s = 0; s < I::FS; ++s) {
-            const int e = tid + s * I::NT;
-            f_base[s] = 0;
-            f_step[s] = 0;
-            if (e < I::NXF) {
-                const int r = e / (TX + 1), fl = e - r * (TX + 1);  // x face f = i0-1+fl, row j0+r
-                f_base[s] = (I::THREE_D ? r + H : 0) * I::LW + fl;
-                f_step[s] = 1;
-            } else if (e < I::NF) {
-                const int e2 = e - I::NXF, fr = e2 / TX, c = e2 - fr * TX;  // y face g = j0-1+fr, column i0+c
-                f_base[s] = fr * I::LW + c + H;
-                f_step[s] = I::LW;
-            }
+            const int ii = wrap(i0 - H + c, A.nx, A.mx), jj = I::THREE_D ? wrap(j0 - H + r, A.ny, A.my) : 1;
+            off[s] = (ii - 1) + A.nx * (jj - 1);
+            pos[s] = e < I::NH ? r * I::LW + c : -1;
         }
     }
 };
 
-// One field marched up the item's levels.  Per level: the prefetched tile
-// goes to LDS, the next level's tile, face velocities, window value and
-// step-start value are requested, every thread evaluates its face slots
-// and the top z face of its column (register window q(k-1..k+2)), then
-// finishes its cell: FP64 flux divergence of the FP32/FP64 face values and
-// the Shu-Osher stage update, rounded once to the field's precision, with
-// the periodic ghost images.
+// One field marched up the item's levels.  Per level the tile goes to LDS (a
+// thread's own value from its column window, the halo as requested one level
+// ahead), every thread forms the west and south face of its cell and the top
+// face of its column (register window q(k-H+1..k+H)), one wave the left-over
+// faces; the faces of the eastern and northern neighbours come through LDS.
+// Then the cell: FP64 flux divergence of the FP32/FP64 face values and the
+// Shu-Osher stage update, rounded once to the field's precision, with the
+// periodic ghost images.
 template <int SCHEME, int TX, int TY, class T>
 __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restrict__ q, const T *__restrict__ q0,
                                             T *__restrict__ out, T *lt, T *lf, const float *lv, int k0, int nk,
                                             int i0, int j0, int tid, int tx, int ty, bool valid, int col,
-                                            const Slots<TX, TY, stencil_h<SCHEME>()> &sl)
+                                            const Halo<TX, TY, stencil_h<SCHEME>()> &halo)
 {
     constexpr int H = stencil_h<SCHEME>();
     using I = Item<TX, TY, H>;
@@ -163,18 +129,22 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
     const bool zdir = (A.dirmask & 4) != 0;
     const int kstart = (k0 > 1 && zdir) ? -1 : 0;
     const int ks = k0 + kstart;
-    // byte offsets in a level plane: this thread's column, its tile slots
-    const uint32_t colb = (uint32_t)col * (uint32_t)sizeof(T);
-    uint32_t tb[I::TS];
+    // byte offsets in a level plane: this thread's column, its halo slots
+    uint32_t colb = (uint32_t)col * (uint32_t)sizeof(T);
+    uint32_t hb[I::HS];
 #pragma unroll
-    for (int s = 0; s < I::TS; ++s) tb[s] = (uint32_t)sl.t_off[s] * (uint32_t)sizeof(T);
+    for (int s = 0; s < I::HS; ++s) hb[s] = (uint32_t)halo.off[s] * (uint32_t)sizeof(T);
+    // own position in the tile, and where the eastern and northern faces lie
+    const int own = (I::THREE_D ? (ty + H) * I::LW : 0) + tx + H;
+    const int fe = tx < TX - 1 ? tid + 1 : I::REST + ty;
+    const int fn = ty < TY - 1 ? I::SOUTH + tid + TX : I::REST + TY + tx;
     // window q(ks-H+1..ks+H), levels outside 1..nz clamped
     T zw[2 * H];
 #pragma unroll
     for (int m = 0; m < 2 * H; ++m) zw[m] = load_at(q + lev(ks - H + 1 + m), colb);
     const float wz0 = load_at(A.w + lev(ks + 1), (uint32_t)col * 4u);
     T fzb = T(0);
-    T tv[I::TS];
+    T hv[I::HS];
     T q0v = T(0), zn = T(0);
     double d1v = 0.0;
     const bool need_q0 = A.epi != 0 && A.c0 != 0.0;
@@ -184,36 +154,63 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
         const size_t kb = lev(k);
         const T *qk = q + kb;
 #pragma unroll
-        for (int s = 0; s < I::TS; ++s)
-            if (sl.t_off[s] >= 0) tv[s] = load_at(qk, tb[s]);
-        if (need_q0 && valid) q0v = load_at(q0 + kb, colb);
+        for (int s = 0; s < I::HS; ++s) hv[s] = load_at(qk, hb[s]);
+        if (need_q0) q0v = load_at(q0 + kb, colb);
         zn = load_at(q + lev(k + H), colb);
         d1v = table(A.dz1w)[k - 1];
     };
     fetch(k0);
+    // waited for here: the waits in the loop then count what a level has in
+    // flight itself, not the fewer requests of the way into it
+#pragma unroll
+    for (int s = 0; s < I::HS; ++s) settle(hv[s]);
+    settle(q0v);
+    settle(zn);
 #pragma unroll 1
     for (int kk = kstart; kk < nk; ++kk) {
         const int k = k0 + kk;
+        // opaque per level: otherwise every array's 64-bit address is hoisted
+        // out of the loop into registers of its own
+#pragma unroll
+        for (int s = 0; s < I::HS; ++s) asm volatile("" : "+v"(hb[s]));
+        asm volatile("" : "+v"(colb));
         // window q(k-H+1..k+H); this level's staged velocities
         const float *lvk = lv + (kk < 0 ? 0 : kk) * I::NV;
-        const T fzt = zdir ? zface<SCHEME, T>(k, nz, zw, T(kk < 0 ? wz0 : lvk[I::NF + tid]), A) : T(0);
+        const T fzt = zdir ? zface<SCHEME, T>(k, nz, zw, T(kk < 0 ? wz0 : lvk[I::NFACE + tid]), A) : T(0);
         if (kk >= 0) {
+            lt[own] = zw[H - 1];
 #pragma unroll
-            for (int s = 0; s < I::TS; ++s)
-                if (sl.t_off[s] >= 0) lt[tid + s * I::NT] = tv[s];
+            for (int s = 0; s < I::HS; ++s)
+                if (halo.pos[s] >= 0) lt[halo.pos[s]] = hv[s];
             const T q0c = q0v;
             const double dz1w_k = d1v;
             __syncthreads();
-            if (kk + 1 < nk) fetch(k + 1);
+            fetch(k0 + min(kk + 1, nk - 1));
+            // a face at a time, each from its own loads: values shared by two
+            // faces would be fused into other multiply-adds in one than in the
+            // other, and the bits would depend on the tile
+            T sv[2 * H], fs = T(0);
 #pragma unroll
-            for (int s = 0; s < I::FS; ++s) {
-                const int st = sl.f_step[s];
-                if (st == 0) continue;
-                const int b = sl.f_base[s];
-                T sv[2 * H];
+            for (int m = 0; m < 2 * H; ++m) sv[m] = lt[own - H + m];
+            T fw = hface<SCHEME, T>(sv, T(lvk[tid]), A, A.dx1);
+            settle(fw);
+            lf[tid] = fw;
+            if constexpr (I::THREE_D) {
+#pragma unroll
+                for (int m = 0; m < 2 * H; ++m) sv[m] = lt[own + (m - H) * I::LW];
+                fs = hface<SCHEME, T>(sv, T(lvk[I::SOUTH + tid]), A, A.dy1);
+                settle(fs);
+                lf[I::SOUTH + tid] = fs;
+            }
+            // the left-over faces, by another wave each level
+            const int lo = (tid + 64 * kk) & (I::NT - 1);
+            if (lo < I::LO) {
+                const bool east = lo < TY;
+                const int b = east ? (I::THREE_D ? (lo + H) * I::LW : 0) + TX : TY * I::LW + lo - TY + H;
+                const int st = east ? 1 : I::LW;
 #pragma unroll
                 for (int m = 0; m < 2 * H; ++m) sv[m] = lt[b + m * st];
-                lf[tid + s * I::NT] = hface<SCHEME, T>(sv, T(lvk[tid + s * I::NT]), A, st == 1 ? A.dx1 : A.dy1);
+                lf[I::REST + lo] = hface<SCHEME, T>(sv, T(lvk[I::REST + lo]), A, east ? A.dx1 : A.dy1);
             }
             __syncthreads();
             if (valid) {
@@ -221,14 +218,8 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
                 // values are exact there, and the three terms are summed
                 // with one rounding per term (a compensated FP32 sum)
                 double div = 0.0;
-                if (A.dirmask & 1) {
-                    const int e = ty * (TX + 1) + tx;
-                    div += (double(lf[e + 1]) - double(lf[e])) * A.dx1;
-                }
-                if (I::THREE_D && (A.dirmask & 2)) {
-                    const int e = I::NXF + ty * TX + tx;
-                    div += (double(lf[e + TX]) - double(lf[e])) * A.dy1;
-                }
+                if (A.dirmask & 1) div += (double(lf[fe]) - double(fw)) * A.dx1;
+                if (I::THREE_D && (A.dirmask & 2)) div += (double(lf[fn]) - double(fs)) * A.dy1;
                 if (A.dirmask & 4) div += (double(fzt) - double(fzb)) * dz1w_k;
                 const double a = -div;
                 T *outk = out + (size_t)(k - 1) * plane;
@@ -267,35 +258,33 @@ __device__ __forceinline__ void march_field(const FusedArgs &A, const T *__restr
     }
 }
 
-// items: work items per group of fpi fields; A.nwork counts all groups' items.
-// T: the precision of every field of the launch (FP64 and FP32 members of
-// a batch go to two launches, so that the FP32 kernel keeps the register
-// budget of FP32 arithmetic).
-// Waves per SIMD the register allocation must allow: six for the FP32
-// 256-thread tiles (see fused_kc).  The other instances are bound by LDS or
-// need their registers (WENO5's six-value stencils among them).
-template <int SCHEME, int TX, int TY, class T>
-constexpr int fused_min_waves()
-{
-    return fused_six_waves<SCHEME, TX, TY, T>() ? 6 : 1;
-}
-
 // LDS of a work item: a field's tile and faces of one level, the chunk's velocities.
 template <int SCHEME, int TX, int TY, class T>
 constexpr int fused_lds_bytes()
 {
     using I = Item<TX, TY, stencil_h<SCHEME>()>;
-    return (I::LH * I::LW + I::FS * I::NT) * (int)sizeof(T) + fused_kc<SCHEME, TX, TY, T>() * I::NV * (int)sizeof(float);
+    return (I::LH * I::LW + I::NFACE) * (int)sizeof(T) + fused_kc<SCHEME, TX, TY, T>() * I::NV * (int)sizeof(float);
 }
 
+// items: work items per group of fpi fields.  T: the precision of every field of the launch (FP64 and FP32 members of
+// a batch go to two launches, so that the FP32 kernel keeps the register
+// budget of FP32 arithmetic).
+//
+// Bound by VALU issue: the FP32 'weno' kernel takes about 190 vector
+// instructions per cell, a third of them the upwind faces it cannot do
+// without, at 85 % of the issue rate (3.6 ms per stage for 15 species at
+// 512x512x160; a copy of its bytes takes 1.7 ms).  Faces by cell instead of a
+// list of faces with their places in registers: constant LDS offsets, one
+// plane offset for all of a thread's loads, 56 registers instead of 80 with
+// spills; 16.0 -> 15.4 ms for a step of 20 fields with the chunks above, eight
+// WENO5 species and two FP64 fields at 192x160x96 420 -> 360 us.
 template <int SCHEME, int TX, int TY, class T>
-__global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(fused_min_waves<SCHEME, TX, TY, T>(), 8))) void
-fused_kernel(FusedArgs A, int items, int fpi)
+__global__ __launch_bounds__(TX *TY) void fused_kernel(FusedArgs A, int items, int fpi)
 {
     constexpr int H = stencil_h<SCHEME>();
     using I = Item<TX, TY, H>;
     __shared__ T tile_lds[I::LH * I::LW];
-    __shared__ T face_lds[I::FS * I::NT];
+    __shared__ T face_lds[I::NFACE];
     constexpr int KC = fused_kc<SCHEME, TX, TY, T>();
     __shared__ float vel_lds[KC * I::NV];
 
@@ -324,66 +313,53 @@ fused_kernel(FusedArgs A, int items, int fpi)
     const bool valid = i <= nx - 2 && (!I::THREE_D || j <= ny - 2);
     const int il = wrap(i, nx, A.mx), jl = I::THREE_D ? wrap(j, ny, A.my) : 1;
     const int col = (il - 1) + nx * (jl - 1);
-    Slots<TX, TY, H> sl;
-    sl.init(tid, i0, j0, A);
-    // the chunk's face velocities and column w(k+1), read once for every
-    // field of the item: the source array and plane offset of each of this
-    // thread's staging slots are fixed, and all the chunk's loads are in
-    // flight together before they go to LDS
+    Halo<TX, TY, H> halo;
+    halo.init(tid, i0, j0, A);
+    // The chunk's face velocities and column w(k+1), read once for every
+    // field: a thread's own west face, south face and column share one
+    // plane offset, the left-over faces go to the first threads.  All the
+    // chunk's loads are in flight together before they go to LDS.
     {
-        constexpr int VS = (I::NV + I::NT - 1) / I::NT;
         const size_t plane = (size_t)nx * ny;
-        const float *vp[VS];
-        int voff[VS];
-        bool vw[VS];
-#pragma unroll
-        for (int s = 0; s < VS; ++s) {
-            const int e = tid + s * I::NT;
-            vp[s] = A.u;
-            voff[s] = -1;
-            vw[s] = false;
-            if (e < I::NF) {
-                int base, step;
-                size_t vcol;
-                const int kind = face_slot_geom<TX, TY, H>(e, i0, j0, A, base, step, vcol);
-                vp[s] = kind == 1 ? A.u : A.v;
-                voff[s] = (int)vcol;
-            } else if (e < I::NV) {
-                const int c = e - I::NF, cx = c % TX, cy = c / TX;
-                const int ci = wrap(i0 + cx, nx, A.mx), cj = I::THREE_D ? wrap(j0 + cy, ny, A.my) : 1;
-                vp[s] = A.w;  // w(k+1) at level k
-                voff[s] = (ci - 1) + nx * (cj - 1);
-                vw[s] = true;
-            }
-        }
-        float vb[KC][VS];
+        const bool rest = tid < I::LO, east = tid < TY;
+        const int ri = wrap(east ? i0 + TX : i0 + tid - TY, nx, A.mx);
+        const int rj = I::THREE_D ? wrap(east ? j0 + tid : j0 + TY, ny, A.my) : 1;
+        const int rcol = (ri - 1) + nx * (rj - 1);
+        const float *rp = east ? A.u : A.v;
+        float vu[KC], vv[KC], vr[KC], vw[KC];
 #pragma unroll
         for (int kk = 0; kk < KC; ++kk) {
             const int k = k0 + kk;
-#pragma unroll
-            for (int s = 0; s < VS; ++s) {
-                vb[kk][s] = 0.0f;
-                if (kk < nk && voff[s] >= 0 && (!vw[s] || k < nz))
-                    vb[kk][s] = vp[s][(size_t)(vw[s] ? k : k - 1) * plane + (size_t)voff[s]];
+            vu[kk] = vv[kk] = vr[kk] = vw[kk] = 0.0f;
+            if (kk < nk) {
+                const size_t kb = (size_t)(k - 1) * plane;
+                vu[kk] = A.u[kb + col];
+                if (I::THREE_D) vv[kk] = A.v[kb + col];
+                if (rest) vr[kk] = rp[kb + rcol];
+                if (k < nz) vw[kk] = A.w[kb + plane + col];  // w(k+1) at level k
             }
         }
 #pragma unroll
         for (int kk = 0; kk < KC; ++kk)
-#pragma unroll
-            for (int s = 0; s < VS; ++s)
-                if (kk < nk && tid + s * I::NT < I::NV) vel_lds[kk * I::NV + tid + s * I::NT] = vb[kk][s];
+            if (kk < nk) {
+                float *l = vel_lds + kk * I::NV;
+                l[tid] = vu[kk];
+                if (I::THREE_D) l[I::SOUTH + tid] = vv[kk];
+                if (rest) l[I::REST + tid] = vr[kk];
+                l[I::NFACE + tid] = vw[kk];
+            }
         __syncthreads();
     }
     if constexpr (sizeof(T) == 8) {
 #pragma unroll 1
         for (int f = f0; f < min(A.n64_active, f0 + fpi); ++f)
             march_field<SCHEME, TX, TY, T>(A, A.q64[f], A.q0_64[f], A.out64[f], tile_lds, face_lds, vel_lds, k0, nk,
-                                           i0, j0, tid, tx, ty, valid, col, sl);
+                                           i0, j0, tid, tx, ty, valid, col, halo);
     } else {
 #pragma unroll 1
         for (int f = f0; f < min(A.n32_active, f0 + fpi); ++f)
             march_field<SCHEME, TX, TY, T>(A, A.q32[f], A.q0_32[f], A.out32[f], tile_lds, face_lds, vel_lds, k0, nk,
-                                           i0, j0, tid, tx, ty, valid, col, sl);
+                                           i0, j0, tid, tx, ty, valid, col, halo);
     }
 }
 

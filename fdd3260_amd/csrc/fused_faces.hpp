@@ -97,22 +97,25 @@ __device__ __forceinline__ T weno_face(T a, T b, T c, T d, T uu, bool nonlin)
 // WENO5-JS (Jiang & Shu 1996) value at the right face of c from a..e =
 // q(i-2..i+2): candidates (2,-7,11)/6, (-1,5,2)/6, (2,5,-1)/6, linear weights
 // 0.1, 0.6, 0.3, smoothness indicators beta_r, eps = 1e-6, p = 2; the
-// divisions are reciprocals.
+// divisions are reciprocals.  The multiply-adds are written out: where both
+// upwind sides share terms, the compiler's choice of them depends on the place the
+// face is evaluated at.
 template <class T>
 __device__ __forceinline__ T weno5_left(T a, T b, T c, T d, T e)
 {
+#pragma clang fp contract(off)
     const T eps = T(1e-6), k13 = T(13.0 / 12.0), sixth = T(1.0 / 6.0);
-    const T q0 = (T(2) * a - T(7) * b + T(11) * c) * sixth;
-    const T q1 = (-b + T(5) * c + T(2) * d) * sixth;
-    const T q2 = (T(2) * c + T(5) * d - e) * sixth;
-    const T s0 = a - T(2) * b + c, t0 = a - T(4) * b + T(3) * c;
-    const T s1 = b - T(2) * c + d, t1 = b - d;
-    const T s2 = c - T(2) * d + e, t2 = T(3) * c - T(4) * d + e;
-    T b0 = eps + (k13 * s0 * s0 + T(0.25) * t0 * t0);
-    T b1 = eps + (k13 * s1 * s1 + T(0.25) * t1 * t1);
-    T b2 = eps + (k13 * s2 * s2 + T(0.25) * t2 * t2);
+    const T q0 = fma(T(11), c, fma(T(-7), b, T(2) * a)) * sixth;
+    const T q1 = fma(T(2), d, fma(T(5), c, -b)) * sixth;
+    const T q2 = fma(T(5), d, fma(T(2), c, -e)) * sixth;
+    const T s0 = fma(T(-2), b, a) + c, t0 = fma(T(3), c, fma(T(-4), b, a));
+    const T s1 = fma(T(-2), c, b) + d, t1 = b - d;
+    const T s2 = fma(T(-2), d, c) + e, t2 = fma(T(3), c, fma(T(-4), d, e));
+    const T b0 = fma(k13 * s0, s0, fma(T(0.25) * t0, t0, eps));
+    const T b1 = fma(k13 * s1, s1, fma(T(0.25) * t1, t1, eps));
+    const T b2 = fma(k13 * s2, s2, fma(T(0.25) * t2, t2, eps));
     const T a0 = T(0.1) * rcp(b0 * b0), a1 = T(0.6) * rcp(b1 * b1), a2 = T(0.3) * rcp(b2 * b2);
-    return (a0 * q0 + a1 * q1 + a2 * q2) * rcp(a0 + a1 + a2);
+    return fma(a2, q2, fma(a1, q1, a0 * q0)) * rcp(a0 + a1 + a2);
 }
 
 // WENO5 face flux from q(f-2..f+3), upwind side only

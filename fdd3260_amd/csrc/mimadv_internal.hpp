@@ -89,7 +89,11 @@ struct AdjArgs {
 
 // Forms v here: keeps the scheduler from overlapping two register-hungry parts
 // of a kernel.
-__device__ __forceinline__ void settle(double &v) { asm volatile("" : "+v"(v) : : "memory"); }
+template <class T>
+__device__ __forceinline__ void settle(T &v)
+{
+    asm volatile("" : "+v"(v) : : "memory");
+}
 
 // Compute units of the current device.
 inline int device_cus()
