@@ -1706,14 +1706,10 @@ FusedArgs multi_args(mimadv_multi *m, int d, double c0, double c1, double dt, in
 // returns the work count in *nwork
 int multi_upload(mimadv_multi *m, std::vector<FusedArgs> &tab, int slot, int *nwork)
 {
-    int begin = 0;
-    for (FusedArgs &A : tab) {
-        multi_prepare(A, begin);
-        begin += A.nwork;
-    }
+    const int work = multi_number(tab);
     MHIPCHK(m, hipMemcpyAsync(m->d_table + (size_t)slot * m->ndom, tab.data(), tab.size() * sizeof(FusedArgs),
                               hipMemcpyHostToDevice, m->stream));
-    *nwork = begin;
+    *nwork = work;
     return MIMADV_OK;
 }
 
@@ -1873,7 +1869,7 @@ int mimadv_multi_autotune(mimadv_multi *m, int reps)
                 m->kchunk[d] = kc;
                 // a middle stage into s2 from q: the fields are only read
                 FusedArgs one = multi_args(m, d, 0.75, 0.25, 1e-3, 0, 2);
-                multi_prepare(one, 0);
+                multi_prepare(one, 0, 1);
                 const int copies = std::min(max_copies, std::max(1, (target + one.nwork - 1) / one.nwork));
                 std::vector<FusedArgs> tab(copies, one);
                 for (int r = 0; r < copies; ++r) tab[r].work_begin = r * one.nwork;

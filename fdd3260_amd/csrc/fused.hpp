@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 namespace mimadv {
 
 constexpr int FUSED_MAX64 = 2;
@@ -33,6 +35,7 @@ struct FusedArgs {
     // multi-domain launches only
     int scheme;        // 0 WENO, 2 MUSCL
     int work_begin;    // first work id of this subdomain in the launch
+    int fpi;           // fields per work item
     int dirmask;  // directions included in the divergence (bit0 x, bit1 y, bit2 z)
 };
 
@@ -46,7 +49,10 @@ hipError_t launch_fused(int scheme, int n64, int n32, const FusedArgs &A, hipStr
 constexpr int MULTI_NT = 256;
 constexpr int MULTI_KC = 6;  // levels of a multi-domain work item (maximum and default)
 bool multi_tile_ok(int tile_x, int tile_y);
-void multi_prepare(FusedArgs &A, int work_begin);  // sets ntx, nty, nwork; kchunk clamped
+// sets ntx, nty, nwork; kchunk clamped; each item marches 1/split of the fields
+void multi_prepare(FusedArgs &A, int work_begin, int split);
+// numbers the work items of a table; returns their count
+int multi_number(std::vector<FusedArgs> &table);
 hipError_t launch_multi(const FusedArgs *d_table, int ndom, int nwork, hipStream_t s);
 
 }  // namespace mimadv

@@ -16,6 +16,7 @@
 // registers and 11.41 ms for three stages of 48 subdomains of 48 to 192 columns a
 // side, the instances 69 and 10.34 ms.)  25 KB of LDS: six groups a CU.
 // Bound by VALU issue, like the single-grid kernel.
+#include <algorithm>
 #include <type_traits>
 
 #include "fused_march.hpp"
@@ -51,9 +52,14 @@ __global__ __launch_bounds__(NT) void multi_kernel(const FusedArgs *__restrict__
     // instead of being reloaded after every store (the table is global
     // memory); the field pointers are read from the table once per field
     const FusedArgs A = table[lo];
-    const int local = wi - A.work_begin;
-    const int tiles = A.ntx * A.nty;
-    const int chunk = local / tiles, t = local - chunk * tiles;
+    // fields f0 .. f1 - 1, level chunk and tile of the item
+    const int tiles = A.ntx * A.nty, nchunk = (A.nz + A.kchunk - 1) / A.kchunk;
+    int t = wi - A.work_begin;
+    const int fg = t / (tiles * nchunk);
+    t -= fg * tiles * nchunk;
+    const int chunk = t / tiles;
+    t -= chunk * tiles;
+    const int f0 = fg * A.fpi, f1 = min(A.n32_active, f0 + A.fpi);
     const auto fields = [&](int f, const float *&q, const float *&q0, float *&out) {
         q = table[lo].q32[f];
         q0 = table[lo].q0_32[f];
@@ -61,13 +67,12 @@ __global__ __launch_bounds__(NT) void multi_kernel(const FusedArgs *__restrict__
     };
     const auto shape = [&](auto scheme) {
         constexpr int S = decltype(scheme)::value;
-        const int nf = A.n32_active;
         if (A.tile_x == 32)
-            march_item<S, 32, 8, float, KC>(A, chunk, t, 0, nf, fields, tile_lds, face_lds, vel_lds);
+            march_item<S, 32, 8, float, KC>(A, chunk, t, f0, f1, fields, tile_lds, face_lds, vel_lds);
         else if (A.tile_x == 16)
-            march_item<S, 16, 16, float, KC>(A, chunk, t, 0, nf, fields, tile_lds, face_lds, vel_lds);
+            march_item<S, 16, 16, float, KC>(A, chunk, t, f0, f1, fields, tile_lds, face_lds, vel_lds);
         else
-            march_item<S, 64, 4, float, KC>(A, chunk, t, 0, nf, fields, tile_lds, face_lds, vel_lds);
+            march_item<S, 64, 4, float, KC>(A, chunk, t, f0, f1, fields, tile_lds, face_lds, vel_lds);
     };
     if (A.scheme == 0) shape(std::integral_constant<int, 0>{});
     else if (A.scheme == 3) shape(std::integral_constant<int, 3>{});
@@ -81,13 +86,35 @@ bool multi_tile_ok(int tile_x, int tile_y)
     return tile_x * tile_y == MULTI_NT && (tile_x == 16 || tile_x == 32 || tile_x == 64);
 }
 
-void multi_prepare(FusedArgs &A, int work_begin)
+void multi_prepare(FusedArgs &A, int work_begin, int split)
 {
     A.ntx = (A.nx - 5 + A.tile_x - 1) / A.tile_x;
     A.nty = (A.ny - 5 + A.tile_y - 1) / A.tile_y;
     A.kchunk = A.kchunk <= 0 ? KC : min(A.kchunk, KC);
-    A.nwork = A.ntx * A.nty * ((A.nz + A.kchunk - 1) / A.kchunk);
+    const int nf = std::max(1, A.n32_active);
+    split = std::min(split, nf);
+    A.fpi = (nf + split - 1) / split;
+    A.nwork = A.ntx * A.nty * ((A.nz + A.kchunk - 1) / A.kchunk) * ((nf + A.fpi - 1) / A.fpi);
     A.work_begin = work_begin;
+}
+
+// Few subdomains leave the chip idle if every item marches all fields: the
+// fields are then split so that the launch has eight groups per CU, as in the
+// single-grid kernel (two subdomains of 48 to 60 columns a side, SSP-RK3 step
+// 455 -> 177 us; from eight groups per CU on nothing is split).
+int multi_number(std::vector<FusedArgs> &table)
+{
+    int work = 0;
+    for (int split = 1;;) {
+        work = 0;
+        for (FusedArgs &A : table) {
+            multi_prepare(A, work, split);
+            work += A.nwork;
+        }
+        if (split > 1 || work == 0) return work;
+        split = (8 * device_cus() + work - 1) / work;
+        if (split <= 1) return work;
+    }
 }
 
 hipError_t launch_multi(const FusedArgs *d_table, int ndom, int nwork, hipStream_t s)

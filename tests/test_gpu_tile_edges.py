@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from fdd3260_amd import Advection
+from fdd3260_amd import Advection, MultiDomain, _lib, cases
 from oracle.oracle import Oracle
 
 from helpers import case2d, case3d
@@ -337,3 +337,31 @@ def test_adjoint_tile_edges(cuda, scheme, dims):
     for n, (x, y) in enumerate(zip(once[1:], twice[1:])):
         scale = max(float(np.abs(x).max()), 1e-300)
         assert float(np.abs(y - 2.0 * x).max()) <= 4 * 2.0 ** -52 * scale, f"velocity {n}"
+
+
+@pytest.mark.parametrize("counts", [(1, 7), (16, 3, 5), (1,), (18, 0, 2, 11, 4, 9)])
+@pytest.mark.parametrize("dims", [(20, 16, 12), (190, 180, 30)])
+def test_multi_field_split(cuda, counts, dims):
+    """Field counts that the split over work items divides and does not, on
+    subdomains too small to fill the chip and large enough, have the bits of
+    a batch of each subdomain."""
+    print(f"case multi_field_split {counts} {dims}", flush=True)
+    advs, vels, fields, refs = [], [], [], []
+    for d, nf in enumerate(counts):
+        g, u, v, w, _ = case3d(*dims, seed=5 + d)
+        rng = np.random.default_rng(40 + d)
+        q = [cases.fill_periodic(g, np.exp(rng.standard_normal(g.shape))).astype(np.float32) for _ in range(nf)]
+        vels.append(tuple(_dev(cuda, *(a.astype(np.float32) for a in (u, v, w)))))
+        fields.append(_dev(cuda, *q))
+        refs.append(_dev(cuda, *q))
+        advs.append(Advection(g, scal_adv=("weno", "muscl", "weno5")[d % 3], muscllimiter="MC"))
+    torch.cuda.synchronize()
+    with MultiDomain(advs, vels, fields) as m:
+        m.advance(_lib.INT_SSPRK3, 2, [0.5] * len(counts))
+    for a, vel, fl, ref in zip(advs, vels, fields, refs):
+        if ref:
+            a.batch_advance(_lib.INT_SSPRK3, 2, 0.5, *vel, ref)
+            a.stream_sync()
+        for n, (x, y) in enumerate(zip(fl, ref)):
+            assert torch.equal(x, y), f"field {n}"
+        a.close()
