@@ -17,8 +17,14 @@
 // k-2..k+1, w at k-1..k+2, columns within two cells of the tile) sit in
 // LDS rings of FP32 tiles with a 2-cell halo, each level loaded once,
 // coalesced; the values read only in the thread's own column (the momenta
-// at k-2, k-1, w at k-2) are carried in registers.  36 KB of LDS per
-// 256-thread group: four groups per CU.  One work item per workgroup.
+// at k-2, k-1, w at k-2) are carried in registers, and so are the z fluxes of
+// u and v, each formed once.  36 KB of LDS per 256-thread group: four groups
+// per CU.  One work item per workgroup.
+//
+// Bound by VALU issue and LDS reads (about 510 vector instructions and 90 LDS
+// reads per cell; the memory traffic takes a third of the time).  A z flux
+// for each of the four cells that use it and loads under lane masks took 560
+// and 113: 887 -> 824 us per stage at 512x512x160.
 #include "mimadv_internal.hpp"
 
 namespace mimadv {
@@ -90,27 +96,36 @@ __device__ __forceinline__ float cross_line(int i, float d1, float d3, const Mom
     return t;
 }
 
-// advuz_fd / advvz_fd with 'nnf' floor and lid (windadv.f90:628-694):
-// W(kk, o) the vertical velocity at level kk and transverse offset o;
-// m2k the level of dz1w on the k = 2 line (1 for u, 2 for v)
+// advuz_fd / advvz_fd with 'nnf' floor and lid (windadv.f90:628-694).
+// Flux of face kk (none through floor and lid), kk in 1..nz-1: M(kk) the
+// momentum, W(kk, o) the vertical velocity at level kk and transverse offset
+// o.  The multiply-adds are written out: a face is evaluated at more than one
+// place, and the bits must not depend on it.
 template <class MF, class WF>
-__device__ __forceinline__ float cross_z(int k, int nz, Table<float> mz, int m2k, const MomF &c, MF M, WF W)
+__device__ __forceinline__ float flux_z(int kk, int nz, Table<float> mz, const MomF &c, MF M, WF W)
+{
+#pragma clang fp contract(off)
+    if (kk >= nz || kk < 1) return 0.0f;
+    const float ww = fmaf(c.c1c, W(kk + 1, -1) + W(kk + 1, 0), -(c.c2c * (W(kk + 1, -2) + W(kk + 1, 1)))) * 0.5f;
+    return ww * fmaf(mz[MOMZ_N * (kk - 1)], M(kk + 1), mz[MOMZ_N * (kk - 1) + 1] * M(kk));
+}
+
+// fm2..fp1: the fluxes of faces k-2..k+1; m2k the level of dz1w on the k = 2
+// line (1 for u, 2 for v)
+template <class MF, class WF>
+__device__ __forceinline__ float cross_z(int k, int nz, Table<float> mz, int m2k, const MomF &c, float fm2, float fm1,
+                                         float f0, float fp1, MF M, WF W)
 {
     auto Zc = [&](int kk, int n) { return mz[MOMZ_N * (kk - 1) + n]; };
-    auto flux = [&](int kk) -> float {
-        if (kk >= nz || kk < 1) return 0.0f;  // 'nnf' lid: Flux(nz) = 0
-        const float ww = (c.c1c * (W(kk + 1, -1) + W(kk + 1, 0)) - c.c2c * (W(kk + 1, -2) + W(kk + 1, 1))) * 0.5f;
-        return ww * (Zc(kk, 0) * M(kk + 1) + Zc(kk, 1) * M(kk));
-    };
     float t;
     if (k >= 3 && k <= nz - 1) {
-        t = c.c1c * (flux(k) - flux(k - 1)) * Zc(k, 2) - c.c2c * (flux(k + 1) - flux(k - 2)) * Zc(k, 4);
+        t = c.c1c * (f0 - fm1) * Zc(k, 2) - c.c2c * (fp1 - fm2) * Zc(k, 4);
     } else if (k == 1) {
-        t = flux(1) * Zc(1, 2);
+        t = f0 * Zc(1, 2);
     } else if (k == 2) {
-        t = c.c1c * (flux(2) - flux(1)) * Zc(m2k, 2) - c.c2c * flux(3) * Zc(2, 4);
+        t = c.c1c * (f0 - fm1) * Zc(m2k, 2) - c.c2c * fp1 * Zc(2, 4);
     } else {
-        t = -flux(nz - 1) * Zc(nz, 2);
+        t = -fm1 * Zc(nz, 2);
     }
     if (c.lavisc && k >= 3 && k <= nz - 2) {
         const float mu = 0.25f * fabsf(W(k, -1) + W(k, 0) + W(k + 1, -1) + W(k + 1, 0)) * Zc(k, 2);
@@ -204,12 +219,14 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
         const bool valid = i <= nx - 2 && (!THREE_D || j <= ny - 2);
         // ring position of this thread's own column
         const int own = (THREE_D ? (ty + H) * LW : 0) + tx + H;
-        // plane offset of ring entry s of this thread (ghost columns read as
+        // plane offsets of this thread's ring entries (ghost columns read as
         // the caller filled them; positions past the array, the padding of a
-        // partial tile, take a periodic image that feeds no interior cell)
-        auto t_off = [&](int s) -> int {
-            const int e = tid + s * NT;
-            if (e >= PL) return -1;
+        // partial tile, take a periodic image that feeds no interior cell;
+        // slots past the ring load their first entry)
+        unsigned toff[TS];
+#pragma unroll
+        for (int s = 0; s < TS; ++s) {
+            const int e = tid + s * NT < PL ? tid + s * NT : 0;
             const int r = e / LW, cc = e - r * LW;
             int ii = i0 - H + cc;
             if (ii > nx) ii = (ii - 4) % mx + 4;
@@ -218,23 +235,18 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                 jj = j0 - H + r;
                 if (jj > ny) jj = (jj - 4) % my + 4;
             }
-            return (ii - 1) + nx * (jj - 1);
-        };
+            toff[s] = (unsigned)((ii - 1) + nx * (jj - 1));
+        }
         // level km of the momenta and w, level kh of the horizontal
-        // velocities (levels outside 1..nz read as zero)
+        // velocities; levels outside 1..nz, which no closure reads, are
+        // replaced by the nearest one
         float pre[6][TS];
         auto fetch = [&](int km, int kh) {
-            const bool inm = km >= 1 && km <= nz, inh = kh >= 1 && kh <= nz;
-            const size_t kbm = inm ? sz * (km - 1) : 0, kbh = inh ? sz * (kh - 1) : 0;
+            const size_t kbm = sz * (min(max(km, 1), nz) - 1), kbh = sz * (min(max(kh, 1), nz) - 1);
 #pragma unroll
-            for (int s = 0; s < TS; ++s) {
-                const int off = t_off(s);
+            for (int s = 0; s < TS; ++s)
 #pragma unroll
-                for (int n = 0; n < 6; ++n) {
-                    const bool h = n == 3 || n == 4;
-                    pre[n][s] = (off >= 0 && (h ? inh : inm)) ? src[n][(h ? kbh : kbm) + off] : 0.0f;
-                }
-            }
+                for (int n = 0; n < 6; ++n) pre[n][s] = (src[n] + (n == 3 || n == 4 ? kbh : kbm))[toff[s]];
         };
         auto store = [&](int km, int kh, bool with_h) {
             const int sm = (km + 6) % 3;
@@ -272,18 +284,34 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             mk1_2 = ringm[2][a1][own];
         }
         wkm2 = ringw[(k0 - 2) & 3][own];
+        // z fluxes of u and v at faces k-2..k+1, carried up the column
+        float fzu[4] = {0.0f, 0.0f, 0.0f, 0.0f}, fzv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const auto face_z = [&](int kk) __attribute__((always_inline)) {
+            const float u = flux_z(kk, nz, mz, c, [&](int lev) { return ringm[0][(lev + 6) % 3][own]; },
+                                   [&](int lev, int o) { return ringw[lev & 3][own + o]; });
+            float v = 0.0f;
+            if (THREE_D)
+                v = flux_z(kk, nz, mz, c, [&](int lev) { return ringm[1][(lev + 6) % 3][own]; },
+                           [&](int lev, int o) { return ringw[lev & 3][own + o * LW]; });
+            fzu[kk - k0 + 2] = u;
+            fzv[kk - k0 + 2] = v;
+        };
+        face_z(k0 - 2);
+        face_z(k0 - 1);
         __syncthreads();
         fetch(k0 + 1, k0 + 1);
         store(k0 + 1, k0 + 1, false);
+        __syncthreads();
+        face_z(k0);
         fetch(k0 + 2, k0 + 1);
+        const unsigned col = (unsigned)(min(i, nx) - 1 + nx * (THREE_D ? min(j, ny) - 1 : 0));
         // step-start momenta of the thread's cell, requested one level ahead
-        const bool need_m0 = valid && a.epi != 0 && a.c0 != 0.0;
+        const bool need_m0 = a.epi != 0 && a.c0 != 0.0;
         float m0n[3] = {0.0f, 0.0f, 0.0f};
         auto fetch_m0 = [&](int kk) {
-            const size_t id = (size_t)(i - 1) + sy * (j - 1) + sz * (kk - 1);
 #pragma unroll
             for (int n = 0; n < 3; ++n)
-                if (n != 1 || THREE_D) m0n[n] = a.m0[n][id];
+                if (n != 1 || THREE_D) m0n[n] = (a.m0[n] + sz * (kk - 1))[col];
         };
         if (need_m0) fetch_m0(k0);
 #pragma unroll 1
@@ -291,10 +319,8 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             store(k + 2, k + 1, true);
             const float m0v[3] = {m0n[0], m0n[1], m0n[2]};
             __syncthreads();
-            if (k < k1) {
-                fetch(k + 3, k + 2);
-                if (need_m0) fetch_m0(k + 1);
-            }
+            fetch(k + 3, k + 2);
+            if (need_m0) fetch_m0(min(k + 1, k1));
             // ring slot of the momenta at level k
             const int s0 = k % 3;
             if (valid) {
@@ -325,7 +351,10 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                     if (THREE_D)
                         t += cross_line(0, c.dy1, c.dy3, c, [&](int dj) { return R(0, 0, dj, k); },
                                         [&](int dj, int o) { return R(4, o, dj, k); });
-                    t += cross_z(k, nz, mz, 1, c, [&](int kk) { return R(0, 0, 0, kk); },
+                    fzu[3] = flux_z(k + 1, nz, mz, c, [&](int kk) { return R(0, 0, 0, kk); },
+                                    [&](int kk, int o) { return R(5, o, 0, kk); });
+                    t += cross_z(k, nz, mz, 1, c, fzu[0], fzu[1], fzu[2], fzu[3],
+                                 [&](int kk) { return R(0, 0, 0, kk); },
                                  [&](int kk, int o) { return R(5, o, 0, kk); });
                     L[0] = t;
                 }
@@ -336,7 +365,10 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                                          [&](int di, int o) { return R(3, di, o, k); });
                     t += self_line(0, c.dy1, c.dy2, c, [&](int dj) { return R(1, 0, dj, k); },
                                    [&](int dj) { return R(4, 0, dj, k); });
-                    t += cross_z(k, nz, mz, 2, c, [&](int kk) { return R(1, 0, 0, kk); },
+                    fzv[3] = flux_z(k + 1, nz, mz, c, [&](int kk) { return R(1, 0, 0, kk); },
+                                    [&](int kk, int o) { return R(5, 0, o, kk); });
+                    t += cross_z(k, nz, mz, 2, c, fzv[0], fzv[1], fzv[2], fzv[3],
+                                 [&](int kk) { return R(1, 0, 0, kk); },
                                  [&](int kk, int o) { return R(5, 0, o, kk); });
                     L[1] = t;
                 }
@@ -382,6 +414,11 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                         }
                     }
                 }
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                fzu[m] = fzu[m + 1];
+                fzv[m] = fzv[m + 1];
             }
             // own-column registers for level k+1; the next level's stores
             // overwrite the slots of the momenta at k and of w at k-1
