@@ -39,15 +39,16 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch (per stage for the batched workloads) of the dominant
+# HBM bytes per launch (per field and stage for the plain path, per stage for
+# the batched workloads) of the dominant
 # kernels, measured with rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of
 # this script, each counter scaled by what it reads for a 256 MiB device copy
 # (--copy-probe 256: FETCH_SIZE counts half the bytes read, WRITE_SIZE all
 # bytes written).  Reported only for the exact configuration measured.
 HBM_TRAFFIC = {
-    ("plain", "256,256,128", "weno", "heun", 2): 551.2e6,
-    ("adjoint", "256,256,128", "weno", "ssprk3", 1): 1078.2e6,
-    ("fused", "f32", "512,512,160", "weno", "ssprk3", 20): 13.542e9,
+    ("plain", "256,256,128", "weno", "heun", 2): 565.0e6,
+    ("adjoint", "256,256,128", "weno", "ssprk3", 1): 1188.5e6,
+    ("fused", "f32", "512,512,160", "weno", "ssprk3", 20): 10.155e9,
 }
 SCHEME_ID = {"weno": 0, "ppm": 1, "muscl": 2, "weno5": 3, "quick": 4, "lw": 5}
 
@@ -637,7 +638,7 @@ def main():
 def plain(args):
     """The 3D plain per-field FP64 forward (256x256x128 by default): the
     log-normal scalar and theta, the reference 'weno' with Heun stages (the
-    reference's integrator), one launch per field and stage, and the other
+    reference's integrator), all fields of a stage in one launch, and the other
     schemes as variants."""
     import torch
 
