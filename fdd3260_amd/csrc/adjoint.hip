@@ -517,7 +517,7 @@ hipError_t launch_tile(AdjArgs A, int per_cu, hipStream_t s)
     // levels.  Chunks of 16 levels -> this rule, two SSP-RK3 steps: 'weno'
     // 24x24x16 334 -> 103 us, 96x96x48 411 -> 230, 139x117x75 503 -> 461,
     // 192x160x96 876 -> 753; WENO5 560 -> 148, 675 -> 398, 1015 -> 820.
-    if (A.kchunk <= 0) A.kchunk = levels_by_rounds(A.nz, (long)A.ntx * A.nty, per_cu, 2);
+    if (A.kchunk <= 0) A.kchunk = levels_by_rounds(A.nz, (long)A.ntx * A.nty, per_cu, 2, A.nz);
     A.kchunk = min(A.kchunk, A.nz);
     const int nchunk = (A.nz + A.kchunk - 1) / A.kchunk;
     A.nwork = A.ntx * A.nty * nchunk;

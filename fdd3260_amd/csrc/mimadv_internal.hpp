@@ -118,16 +118,16 @@ inline int levels_per_item(int nz, long tiles, int per_cu, int most)
 }
 
 // Levels per work item where starting an item costs as much as `fill` levels:
-// items run in rounds of per_cu groups per CU, so the length with the least
-// rounds * (levels + fill) is taken, the longest of equals.  Small grids get
-// short items on all CUs, and tiles that fill a round and a part of one are
-// cut until the rounds are nearly full.
-inline int levels_by_rounds(int nz, long tiles, int per_cu, int fill)
+// items run in rounds of per_cu groups per CU, so the length of at most `most`
+// levels with the least rounds * (levels + fill) is taken, the shortest of
+// equals.  Small grids get short items on all CUs, and tiles that fill a round
+// and a part of one are cut until the rounds are nearly full.
+inline int levels_by_rounds(int nz, long tiles, int per_cu, int fill, int most)
 {
     const long slots = (long)per_cu * device_cus();
-    int levels = nz;
+    int levels = 1;
     long best = 0;
-    for (int k = nz; k >= 1; --k) {
+    for (int k = 1; k <= std::min(nz, most); ++k) {
         const long rounds = (tiles * ((nz + k - 1) / k) + slots - 1) / slots;
         if (best == 0 || rounds * (k + fill) < best) {
             best = rounds * (k + fill);

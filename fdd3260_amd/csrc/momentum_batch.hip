@@ -465,7 +465,7 @@ hipError_t launch_momentum_batch(const GridDev &g, int mom_ord, int lavisc, cons
     // which are 4 % faster than 16-level ones).  Whole columns or at least 32
     // levels -> this rule: 20 fields at 96x96x48 (36 tiles) 301 -> 196 us, at
     // 192x160x96 (120) 531 -> 468 us, 8 fields at 400x400x100 (650) 1121 -> 1049 us.
-    const int kchunk = levels_by_rounds(g.nz, tiles, three_d ? 4 : 16, 2);
+    const int kchunk = levels_by_rounds(g.nz, tiles, three_d ? 4 : 16, 2, g.nz);
     const int nchunk = (g.nz + kchunk - 1) / kchunk;
     if (three_d) {
         constexpr int TX = 32, TY = 8;

@@ -33,6 +33,8 @@ namespace {
 // full divisions in the limiter (1670 vector instructions per cell, now 760):
 // 256x256x128 430 -> 280 us, 139x117x75 96 -> 63 us, 128x128 (2D) 11.6 -> 10.3
 // us.  32x8 tiles take 314 us, 144 VGPRs without spills (three groups) 300 us.
+// (228 us per field at 256x256x128 since the level metrics are scalar loads and
+// two fields share a launch.)
 template <int TX, int TY>
 __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 8))) void ppm_march_kernel(
     GridDev g, SchemeParams sp, ScalarList l, int kchunk, int ntx)
@@ -346,7 +348,12 @@ template <int TX, int TY>
 hipError_t launch_ppm(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, int per_cu, hipStream_t s)
 {
     const int ntx = (g.nx - 5 + TX - 1) / TX, nty = TY > 1 ? (g.ny - 5 + TY - 1) / TY : 1;
-    const int kchunk = levels_per_item(g.nz, (long)ntx * nty * nf, per_cu, 16);
+    // a chunk's start costs about one level; sixteen levels at most (longer
+    // ones lose the planes of the level above from L2: 456 -> 537 us for two
+    // fields at 256x256x128 with 25).  At most as many items as fit one round
+    // -> this rule, Heun step: 300x200x100 474 -> 422 us, 190x131x75 (two
+    // fields) 349 -> 300 us.
+    const int kchunk = levels_by_rounds(g.nz, (long)ntx * nty * nf, per_cu, 1, 16);
     const int items = ntx * nty * ((g.nz + kchunk - 1) / kchunk);
     hipLaunchKernelGGL((ppm_march_kernel<TX, TY>), dim3(items, nf), dim3(TX * TY), 0, s, g, sp, a, kchunk, ntx);
     return hipGetLastError();
@@ -355,8 +362,6 @@ hipError_t launch_ppm(const GridDev &g, const SchemeParams &sp, const ScalarList
 hipError_t launch_list(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, hipStream_t s)
 {
     switch (sp.scheme) {
-    // one round of the resident groups: two rounds take 67 instead of 63 us at
-    // 139x117x75 and the same at 256x256x128
     case 1: return g.ny > 1 ? launch_ppm<16, 16>(g, sp, a, nf, 4, s) : launch_ppm<64, 1>(g, sp, a, nf, 16, s);
     case 0: case 2: case 3: case 4: case 5: case 6: case 7: return launch_march(g, sp, a, nf, s);
     default: return hipErrorInvalidValue;

@@ -531,21 +531,25 @@ hipError_t launch_tile(const GridDev &g, const SchemeParams &sp, const ScalarLis
 //
 // Levels per item: a level is a serial chain of loads, faces and two barriers
 // (4 us in 3D, 2.4 us on the single-wave 2D tiles), so short chunks on all CUs
-// beat long ones on a few; the start of a chunk costs about one level.  32x8
-// tiles take one round of the four resident groups per CU, at most 8 levels:
-// 'weno' 55 -> 13 us at 64x64x48 (1 level; 8 before), 67 -> 41 us at
-// 139x117x75 (6), unchanged at 256x256x128 (8).  WENO5's longer levels are
-// better balanced by two rounds: 113 -> 64 us at 139x117x75 (3 levels; 16
-// before; one round takes 68).  2D tiles are one wave each, 16 per CU: 38 -> 7
-// us at 128x128 (1 level; 16 before).
+// beat long ones on a few; the start of a chunk costs about one level.  The
+// items of all fields run in rounds of the four resident groups per CU, and the
+// length with the least rounds * (levels + 1) is taken, sixteen levels at most
+// (longer ones lose the planes of the level above from L2).  'weno' 55 -> 13
+// us at 64x64x48 (1 level; 8 before), 67 -> 41 us at 139x117x75 (6).  Against
+// at most eight levels and as many items as fit one round, Heun step: two
+// fields at 256x256x128 590 -> 578 us (16), at 139x117x75 144 -> 138 us (6),
+// one at 300x200x100 253 -> 244 us (13), MUSCL there 278 -> 263 us.
+// WENO5's longer levels are better balanced by at most eight items per CU: 113 -> 64
+// us at 139x117x75 (3 levels; 16 before), least rounds take 71.  2D tiles are
+// one wave each, 16 per CU: 38 -> 7 us at 128x128 (1 level; 16 before).
 template <int S, int TX3, int TY3>
 hipError_t launch_dims(const GridDev &g, const SchemeParams &sp, const ScalarList &a, int nf, hipStream_t s)
 {
-    constexpr int MOST = 8;
-    const long ntx3 = (g.nx - 5 + TX3 - 1) / TX3, nty3 = (g.ny - 5 + TY3 - 1) / TY3;
+    const long tiles = (g.nx - 5 + TX3 - 1) / TX3 * ((g.ny - 5 + TY3 - 1) / TY3) * (long)nf;
     if (g.ny > 1)
-        return launch_tile<TX3, TY3, S>(g, sp, a, nf, levels_per_item(g.nz, ntx3 * nty3 * nf, S == 3 ? 8 : 4, MOST), s);
-    return launch_tile<64, 1, S>(g, sp, a, nf, levels_per_item(g.nz, (g.nx - 5 + 63) / 64 * nf, 16, MOST), s);
+        return launch_tile<TX3, TY3, S>(
+            g, sp, a, nf, S == 3 ? levels_per_item(g.nz, tiles, 8, 8) : levels_by_rounds(g.nz, tiles, 4, 1, 16), s);
+    return launch_tile<64, 1, S>(g, sp, a, nf, levels_by_rounds(g.nz, (g.nx - 5 + 63) / 64 * (long)nf, 16, 1, 16), s);
 }
 
 }  // namespace
