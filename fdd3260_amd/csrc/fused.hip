@@ -65,9 +65,9 @@ constexpr int fused_lds_bytes()
 // a batch go to two launches, so that the FP32 kernel keeps the register
 // budget of FP32 arithmetic).
 //
-// Bound by VALU issue: the FP32 'weno' kernel takes about 190 vector
-// instructions per cell, a third of them the upwind faces it cannot do
-// without, at 85 % of the issue rate (3.6 ms per stage for 15 species at
+// Bound by VALU issue: the FP32 'weno' kernel takes 196 vector instructions
+// per cell, three quarters of them the upwind faces, at 99 % of the issue
+// rate of the clock it runs at (3.6 ms per stage for 15 species at
 // 512x512x160; a copy of its bytes takes 1.7 ms).  Faces by cell instead of a
 // list of faces with their places in registers: constant LDS offsets, one
 // plane offset for all of a thread's loads, 56 registers instead of 80 with

@@ -21,10 +21,11 @@
 // u and v, each formed once.  36 KB of LDS per 256-thread group: four groups
 // per CU.  One work item per workgroup.
 //
-// Bound by VALU issue and LDS reads (about 510 vector instructions and 90 LDS
-// reads per cell; the memory traffic takes a third of the time).  A z flux
-// for each of the four cells that use it and loads under lane masks took 560
-// and 113: 887 -> 824 us per stage at 512x512x160.
+// Bound by VALU issue and LDS reads (478 vector instructions, 69 % of the
+// issue slots, and 101 LDS operations per cell; the memory traffic takes a
+// third of the time).  A z flux for each of the four cells that use it and
+// loads under lane masks took 562 and 113: 887 -> 824 us per stage at
+// 512x512x160.
 #include "mimadv_internal.hpp"
 
 namespace mimadv {
