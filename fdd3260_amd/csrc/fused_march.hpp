@@ -27,10 +27,10 @@ struct Item {
 };
 
 // This thread's part of the halo of a work item's tile, the same for every
-// field and level: offsets in a level plane (32 bits; threads past the end of the list
-// load their own column) and in the LDS tile.  The list holds the H columns west and east of
-// every row, then the H rows south and north of every column; no face reads a
-// corner.
+// field and level: offsets in a level plane (32 bits; threads past the end of
+// the list load its last value) and in the LDS tile (-1 past the end).  The
+// list holds the H columns west and east of every row, then the H rows south
+// and north of every column; no face reads a corner.
 template <int TX, int TY, int H>
 struct Halo {
     using I = Item<TX, TY, H>;

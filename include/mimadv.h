@@ -329,7 +329,7 @@ int mimadv_batch_budget_device(mimadv_ctx *ctx, int nf, const int *precision, co
  * and 'nnf' vertical boundaries, scheme MIMADV_WENO, MIMADV_WENO5 or MIMADV_MUSCL, 3D),
  * its FP32 velocity (u[d], v[d], w[d]) and nf[d] FP32 fields q[d][0..nf-1]
  * (device arrays, at most 18 per subdomain).  Every stage of every
- * subdomain is one work list of one persistent launch; the tile shape
+ * subdomain is one work list of one launch; the tile shape
  * (tile_x * tile_y = 256 with tile_x in 16, 32, 64) and the level
  * chunk are chosen per subdomain.  The plan keeps two stage arrays per
  * field and runs on the stream of ctx[0]. */
